@@ -309,6 +309,31 @@ int hif8_transpose_bf16(const uint16_t *x, int64_t rows, int64_t cols, int64_t r
 int hif8_linear_wgrad(const uint16_t *g, const uint16_t *x, uint16_t *dw, int64_t tokens, int64_t n_out,
                       int64_t k_in, void *workspace, int64_t workspace_bytes, hif8_stream_t stream);
 
+/* Workspace of a wider split: as hif8_linear_split_workspace_bytes, and k ranges also for the grids
+ * that leaves whole although they idle CUs (fewer tiles than CUs, or a last wave over half full), where
+ * the time they save exceeds the partials' traffic.  hif8_linear_wgrad, hif8_linear_fwd_wq_split and
+ * the two entry points below split so when the workspace holds that many bytes (at most 192 MiB on
+ * 256 CUs; the 36 tiles of the 1.3B q/k/v/o weight gradient split 7 ways). */
+int64_t hif8_linear_ksplit_workspace_bytes(int64_t M, int64_t N, int64_t K);
+
+/* The backward's products (hif8_linear.py:97,104) where the reference holds one operand in fp32, its
+ * quantised values x_q = decode(code) / scale: with that operand given as the HiF8 values themselves,
+ * v = decode(code) (hif8_decode_values; exact in bf16),
+ *   hif8_linear_wgrad_scaled: dw[n_out, k_in] = g[tokens, n_out]^T . v[tokens, k_in] / scale
+ *   hif8_linear_fwd_scaled:   y[M, N] = a[M, K] . v[N, K]^T / scale
+ * with fp32 sums of exact products and the scale of the state of the tensor v was encoded from, one
+ * division per output; out_dtype HIF8_DTYPE_F32 or HIF8_DTYPE_BF16 (RNE).  Shapes and alignment as
+ * hif8_linear_wgrad (tokens below 2^22) and hif8_linear_fwd_wq; workspace NULL, or
+ * hif8_linear_ksplit_workspace_bytes (n_out, k_in, tokens or M, N, K) bytes. */
+int hif8_linear_wgrad_scaled(const uint16_t *g, const uint16_t *v, const void *v_state, void *dw, int out_dtype,
+                             int64_t tokens, int64_t n_out, int64_t k_in, void *workspace, int64_t workspace_bytes,
+                             hif8_stream_t stream);
+int hif8_linear_fwd_scaled(const uint16_t *a, const uint16_t *v, const void *v_state, void *y, int out_dtype,
+                           int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes,
+                           hif8_stream_t stream);
+/* The HiF8 values of codes, y = decode(code) in bf16 (exact); y 16-byte aligned. */
+int hif8_decode_values(const uint8_t *codes, int64_t n, uint16_t *y, hif8_stream_t stream);
+
 /* The backward's products for a layer that computes in fp32: grad_q @ w_q and grad_q^T @ x_q
  * (hif8_linear.py:97,104), which the reference evaluates as matmuls in the saved tensors' dtype.
  *   c[m][n] = sum_k a[m*sa_m + k*sa_k] * b[k*sb_k + n*sb_n]      (fp32 fused multiply-adds)

@@ -1075,6 +1075,11 @@ int hif8_decode(const uint8_t *codes, int64_t n, const void *state, int out_dtyp
     return launch_quant(codes, out_dtype, n, state, y, 2, HIF8_SEM_NPU, 1, stream);
 }
 
+int hif8_decode_values(const uint8_t *codes, int64_t n, uint16_t *y, hif8_stream_t stream)
+{
+    return launch_quant(codes, HIF8_DTYPE_BF16, n, nullptr, y, 2, HIF8_SEM_NPU, 0, stream);
+}
+
 int hif8_quant_f32(const float *x, float *y, int64_t n, int semantics, hif8_stream_t stream)
 {
     return launch_quant(x, HIF8_DTYPE_F32, n, nullptr, y, 1, semantics, 0, stream);

@@ -1,7 +1,7 @@
 // The GEMMs of HIF8Linear off the bf16 MFMA path (MI355X, gfx950):
-//   - k_gemm_f32: C = A . B with fp32 accumulation on strided bf16 or fp32 operands -- the
-//     backward's grad_q @ w_q and grad_q^T @ x_q (ospnext/modules/hif8_linear.py:97,104) of a
-//     layer that computes in fp32 (the reference's matmuls run in the saved tensors' dtype);
+//   - k_gemm_f32: C = A . B with fp32 accumulation on strided bf16 or fp32 operands -- the fp32
+//     products of QLinear, and HIF8Linear's backward with an fp32 operand where the operands are
+//     beyond the 32-bit offsets of the MFMA route (hif8_gemm_scaled.hip);
 //   - k_pad_2d: zero padding (or cropping) of a row-major matrix, so that shapes outside the
 //     MFMA kernels' tiles (in_features % 64 != 0, out_features % 8 != 0) run on those kernels
 //     over zero-padded operands (zero codes decode to 0, zero rows and columns add nothing).

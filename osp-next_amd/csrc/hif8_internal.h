@@ -62,6 +62,22 @@ int launch_linear_w16(const uint16_t *x, const uint16_t *w_q, const uint16_t *bi
                       int64_t N, int64_t K, hif8_stream_t stream, State *y_st, float y_smax);
 int launch_linear_w16_groups(const uint16_t *x, const uint16_t *w_q, const Groups &g, const uint16_t *bias,
                              int64_t M, int64_t N, int64_t K, hif8_stream_t stream);
+// The GEMM's tiles of 256 x 256 outputs as whole tiles and, from tile `full` on, `tail` tiles of
+// `splits` k ranges each (splits 1: none), whose fp32 sums a reduce kernel adds in range order.
+struct SplitPlan {
+    int full;     // tiles computed whole
+    int tail;     // tiles computed in k ranges
+    int splits;   // k ranges per tail tile (1: no split)
+    int64_t bytes() const { return splits > 1 ? int64_t(tail) * splits * 256 * 256 * 4 : 0; }
+};
+// plan_split's splits, and k ranges for the grids it leaves whole although they idle CUs
+// (hif8_gemm_w16.hip).
+SplitPlan plan_ksplit(int64_t tiles, int64_t K);
+// The fp32 partials of plan's split tiles into part (EPI 2 of the decode-free kernel); tr: k-major
+// operands.
+int launch_w16_partials(const uint16_t *x, const uint16_t *w_q, int64_t M, int64_t N, int64_t K, const SplitPlan &plan,
+                        float *part, bool tr, hif8_stream_t stream);
+
 // The grouped form: N is the total of the groups' features.
 int launch_linear_dtl_groups(const uint16_t *x, const uint8_t *w_codes, const Groups &g, const uint16_t *bias,
                              int64_t M, int64_t N, int64_t K, hif8_stream_t stream);

@@ -15,8 +15,9 @@ Backward (hif8_linear.py:88-111) quantises the incoming gradient with
 ``scale_max_backward`` through the same HIP kernels.  dgrad ``grad_q @ w_q``
 runs on the forward's GEMM against the transposed weight codes, and wgrad
 ``grad_q^T @ x_q`` on the decode-free GEMM reading both operands token-major,
-when the operands are bf16 (the reference's autocast case); an fp32 operand takes
-the library's fp32 GEMM (``hif8_gemm_f32``) on the same dequantised operands.
+when the operands are bf16 (the reference's autocast case); with an x_q or w_q held in
+fp32 the same GEMM takes its HiF8 values and divides the sums by its scale
+(``hif8_linear_wgrad_scaled``, ``hif8_linear_fwd_scaled``).
 Shapes outside the MFMA tiles (in_features % 64, out_features % 8, or the dgrad's
 reduction % 64) run those GEMMs on zero-padded operands (``hif8_pad_2d``).  No
 product runs on a vendor or torch GEMM.
@@ -316,8 +317,7 @@ def linear_wgrad(grad_q2: Tensor, x_q2: Tensor, split_tail: bool = True, transpo
     L = _lib.load()
     if not transposed:
         dw = torch.empty((N, K), dtype=torch.bfloat16, device=g.device)
-        nbytes = int(L.hif8_linear_split_workspace_bytes(N, K, M)) if split_tail else 0
-        ws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=g.device) if nbytes > 0 else None
+        ws, nbytes = _ksplit_workspace(N, K, M, g.device) if split_tail else (None, 0)
         rc = L.hif8_linear_wgrad(g.data_ptr(), x.data_ptr(), dw.data_ptr(), M, N, K,
                                  ws.data_ptr() if ws is not None else None, nbytes, _lib.stream_ptr(g.device))
         if rc != _lib.ERR_SHAPE:
@@ -326,13 +326,79 @@ def linear_wgrad(grad_q2: Tensor, x_q2: Tensor, split_tail: bool = True, transpo
     Mp = (M + 63) // 64 * 64
     g_t = transpose_bf16(g, Mp)
     x_t = transpose_bf16(x, Mp)
-    return linear_fwd_wq_split(g_t, x_t, split_tail=split_tail)
+    return linear_fwd_wq_split(g_t, x_t, split_tail=split_tail, wide=True)
 
 
-def linear_fwd_wq_split(a: Tensor, w_q: Tensor, bias: Optional[Tensor] = None, split_tail: bool = True) -> Tensor:
+def _ksplit_workspace(M: int, N: int, K: int, device: torch.device) -> Tuple[Optional[Tensor], int]:
+    """The fp32 partials of a GEMM's k ranges (hif8_linear_ksplit_workspace_bytes) and their bytes."""
+    nbytes = int(_lib.load().hif8_linear_ksplit_workspace_bytes(M, N, K))
+    return (torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=device) if nbytes > 0 else None), nbytes
+
+
+def decode_values(codes: Tensor) -> Tensor:
+    """The HiF8 values decode(code) of codes, exact in bf16 (hif8_decode_values)."""
+    _lib.require_gpu_tensor(codes, "codes")
+    codes = _aligned(codes)
+    y = torch.empty(codes.shape, dtype=torch.bfloat16, device=codes.device)
+    if codes.numel():
+        _lib.check(_lib.load().hif8_decode_values(codes.data_ptr(), codes.numel(), y.data_ptr(),
+                                                  _lib.stream_ptr(codes.device)), "hif8_decode_values")
+    return y
+
+
+def linear_wgrad_scaled(grad_q2: Tensor, codes: Tensor, state: QuantState, out_dtype: torch.dtype) -> Optional[Tensor]:
+    """grad_q^T [N, M] @ x_q [M, K] -> [N, K] in ``out_dtype`` for a bf16 grad_q and the codes of an x
+    quantised in fp32 (hif8_linear.py:104 with x_q fp32): the MFMA GEMM on the HiF8 values, divided by
+    x's scale (hif8_linear_wgrad_scaled).  Features are zero-padded to multiples of 8.  None for
+    operands beyond its 32-bit offsets."""
+    M, N = grad_q2.shape
+    K = codes.shape[1]
+    Np, Kp = _round_up(N, 8), _round_up(K, 8)
+    g = _aligned(pad_2d(grad_q2.contiguous(), M, Np) if Np != N else grad_q2.contiguous())
+    if Kp != K:
+        codes = pad_2d(codes.contiguous(), M, Kp)
+    v = decode_values(codes)
+    dw = torch.empty((Np, Kp), dtype=out_dtype, device=g.device)
+    ws, nbytes = _ksplit_workspace(Np, Kp, M, g.device)
+    rc = _lib.load().hif8_linear_wgrad_scaled(g.data_ptr(), v.data_ptr(), state.ptr, dw.data_ptr(),
+                                              _lib.dtype_code(out_dtype), M, Np, Kp,
+                                              ws.data_ptr() if ws is not None else None, nbytes,
+                                              _lib.stream_ptr(g.device))
+    if rc == _lib.ERR_SHAPE:
+        return None
+    _lib.check(rc, "hif8_linear_wgrad_scaled")
+    return dw if (Np, Kp) == (N, K) else pad_2d(dw, N, K)
+
+
+def linear_dgrad_scaled(grad_q2: Tensor, w: "PackedWeight", out_dtype: torch.dtype) -> Optional[Tensor]:
+    """grad_q [M, N] @ w_q [N, K] -> [M, K] in ``out_dtype`` for a bf16 grad_q and a weight quantised
+    in fp32 (hif8_linear.py:97 with w_q fp32): the MFMA GEMM on the HiF8 values of the transposed
+    codes, divided by the weight's scale (hif8_linear_fwd_scaled), zero-padded as ``linear_dgrad``
+    is.  None for a reduction beyond the GEMM's range."""
+    M, N = grad_q2.shape
+    K = w.shape[1]
+    Np, Kp = _round_up(N, 64), _round_up(K, 8)
+    g = _aligned(grad_q2.contiguous())
+    if Np != N:
+        g = pad_2d(g, M, Np)
+    v = decode_values(w.codes_t() if (Np, Kp) == (N, K) else w.codes_t_padded(Kp, Np))
+    y = torch.empty((M, Kp), dtype=out_dtype, device=g.device)
+    ws, nbytes = _ksplit_workspace(M, Kp, Np, g.device)
+    rc = _lib.load().hif8_linear_fwd_scaled(g.data_ptr(), v.data_ptr(), w.state.ptr, y.data_ptr(),
+                                            _lib.dtype_code(out_dtype), M, Kp, Np,
+                                            ws.data_ptr() if ws is not None else None, nbytes,
+                                            _lib.stream_ptr(g.device))
+    if rc == _lib.ERR_SHAPE:
+        return None
+    _lib.check(rc, "hif8_linear_fwd_scaled")
+    return y if Kp == K else pad_2d(y, M, K)
+
+
+def linear_fwd_wq_split(a: Tensor, w_q: Tensor, bias: Optional[Tensor] = None, split_tail: bool = True,
+                        wide: bool = False) -> Tensor:
     """hif8_linear_fwd_wq_split: y = a @ w_q^T (+ bias), bf16, with the tail of the tile grid split
-    over k ranges into a transient fp32 workspace (hif8_linear_split_workspace_bytes) unless
-    ``split_tail`` is False."""
+    over k ranges into a transient fp32 workspace (hif8_linear_split_workspace_bytes, or with
+    ``wide`` hif8_linear_ksplit_workspace_bytes) unless ``split_tail`` is False."""
     M, K = a.shape
     N = w_q.shape[0]
     if w_q.shape[1] != K or w_q.dtype != torch.bfloat16 or a.dtype != torch.bfloat16:
@@ -343,7 +409,8 @@ def linear_fwd_wq_split(a: Tensor, w_q: Tensor, bias: Optional[Tensor] = None, s
     if bias is not None:
         bias = bias.detach().to(torch.bfloat16).contiguous()
         b_ptr = bias.data_ptr()
-    nbytes = int(L.hif8_linear_split_workspace_bytes(M, N, K)) if split_tail else 0
+    need = L.hif8_linear_ksplit_workspace_bytes if wide else L.hif8_linear_split_workspace_bytes
+    nbytes = int(need(M, N, K)) if split_tail else 0
     ws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=a.device) if nbytes > 0 else None
     _lib.check(L.hif8_linear_fwd_wq_split(a.data_ptr(), w_q.data_ptr(), b_ptr, y.data_ptr(), M, N, K,
                                           ws.data_ptr() if ws is not None else None, nbytes,
@@ -682,25 +749,33 @@ class _HIF8LinearFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         # x_q and w_q as the reference saves them (hif8_linear.py:78-82)
-        if ctx.a_fmt == _lib.A_CODES:
-            x_q = decode(ctx.a, ctx.a_st, torch.bfloat16 if ctx.x_dtype == torch.bfloat16 else torch.float32)
-        else:
-            x_q = ctx.a
         grad_q, _ = _quant(grad_output.contiguous(), ctx.smb)            # :93
         g_2d = grad_q.reshape(-1, grad_q.shape[-1]).contiguous()
         M, N = g_2d.shape
         K = ctx.packed.shape[1]
+        g_bf16 = g_2d.dtype == torch.bfloat16
         if dgrad_fused_ok(g_2d, ctx.packed):                              # :97, grad_q @ w_q
             grad_input = linear_dgrad(g_2d, ctx.packed)
-        else:                                                             # fp32: the fp32 GEMM
-            w_q = ctx.packed.dequantize(ctx.w_dtype)                      # [N, K]
-            grad_input = gemm_f32(g_2d, w_q, M, K, N, (N, 1), (K, 1))
+        else:                                                             # w_q fp32
+            grad_input = None
+            if g_bf16 and ctx.packed.src_dtype == ctx.w_dtype == torch.float32:
+                grad_input = linear_dgrad_scaled(g_2d, ctx.packed, ctx.x_dtype)
+            if grad_input is None:
+                w_q = ctx.packed.dequantize(ctx.w_dtype)                  # [N, K]
+                grad_input = gemm_f32(g_2d, w_q, M, K, N, (N, 1), (K, 1))
         grad_input = grad_input.to(ctx.x_dtype).view(ctx.x_shape)
-        x_2d = x_q.reshape(-1, x_q.shape[-1]).contiguous()
-        if wgrad_ok(g_2d, x_2d):                                            # :104, g^T @ x_q
-            grad_weight = linear_wgrad(g_2d, x_2d).to(ctx.w_dtype)
-        else:                                                               # g[M, N]^T x[M, K]
-            grad_weight = gemm_f32(g_2d, x_2d, N, K, M, (1, N), (K, 1)).to(ctx.w_dtype)
+        grad_weight = None                                                # :104, g^T @ x_q
+        if ctx.a_fmt == _lib.A_CODES and ctx.x_dtype != torch.bfloat16 and g_bf16:   # x_q fp32
+            grad_weight = linear_wgrad_scaled(g_2d, ctx.a.reshape(M, K), ctx.a_st, ctx.w_dtype)
+        if grad_weight is None:
+            x_q = ctx.a
+            if ctx.a_fmt == _lib.A_CODES:
+                x_q = decode(ctx.a, ctx.a_st, torch.bfloat16 if ctx.x_dtype == torch.bfloat16 else torch.float32)
+            x_2d = x_q.reshape(-1, x_q.shape[-1]).contiguous()
+            if wgrad_ok(g_2d, x_2d):
+                grad_weight = linear_wgrad(g_2d, x_2d).to(ctx.w_dtype)
+            else:                                                         # g[M, N]^T x[M, K]
+                grad_weight = gemm_f32(g_2d, x_2d, N, K, M, (1, N), (K, 1)).to(ctx.w_dtype)
         grad_bias = g_2d.sum(0).to(ctx.b_dtype) if ctx.has_bias else None                   # :107
         return grad_input, grad_weight, grad_bias, None, None, None, None
 
