@@ -478,6 +478,20 @@ int hif8_attention_fwd(const uint16_t *q, const uint16_t *k, const uint16_t *v, 
                        const int32_t *key_count, float softmax_scale, void *out_state, int out_state_dtype,
                        float scale_max, hif8_stream_t stream);
 
+/* hif8_attention_fwd with the last wave of query tiles (384 queries of one batch and head each, one
+ * workgroup per CU) computed as key ranges where that ends sooner: a second kernel adds the ranges'
+ * fp32 partials in a fixed order, so the result is deterministic and within fp32 rounding of the
+ * unsplit one.  The workspace is hif8_attention_workspace_bytes(batch, n_q, n_kv, heads) bytes of device
+ * memory, 16-byte aligned (at most 150 MB on 256 CUs; 0 where nothing is split); workspace NULL is
+ * hif8_attention_fwd.  Sequences of any length, key lists, counts and states as there. */
+int64_t hif8_attention_workspace_bytes(int64_t batch, int64_t n_q, int64_t n_kv, int64_t heads);
+int hif8_attention_fwd_split(const uint16_t *q, const uint16_t *k, const uint16_t *v, uint16_t *out, int64_t batch,
+                             int64_t n_q, int64_t n_kv, int64_t heads, int64_t head_dim, const int64_t *row_strides,
+                             const int64_t *batch_strides, const int32_t *key_idx, int64_t idx_batch_stride,
+                             const int32_t *key_count, float softmax_scale, void *out_state, int out_state_dtype,
+                             float scale_max, void *workspace, int64_t workspace_bytes, hif8_stream_t stream);
+
+
 #ifdef __cplusplus
 }
 #endif

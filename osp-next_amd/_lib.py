@@ -70,6 +70,9 @@ SIGNATURES = {
     "hif8_rms_norm_rope_fake_quant": (_i, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _f, _p, _i, _p, _p, _p]),
     "hif8_attention_fwd": (_i, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64),
                                 ctypes.POINTER(_i64), _p, _i64, _p, _f, _p, _i, _f, _p]),
+    "hif8_attention_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64]),
+    "hif8_attention_fwd_split": (_i, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64),
+                                      ctypes.POINTER(_i64), _p, _i64, _p, _f, _p, _i, _f, _p, _i64, _p]),
 }
 
 _lib = None

@@ -41,6 +41,7 @@
 //     which the traffic is 2 % (a copy loading the same 64 L2-resident rows every tile) and the
 //     rest their issue and LDS writes: loading two tiles ahead into three buffers was slower, and
 //     without the per-tile barrier the kernel ran the same (measured by removing each).
+//   - A last wave of few tiles runs as key ranges whose partials k_attn_combine adds (plan_split).
 //   - Tile order: workgroup w runs on XCD w % 8; consecutive query tiles of one head are given to
 //     one XCD, so the CUs of an XCD stream the same K/V tiles through its L2.
 #include <hip/hip_runtime.h>
@@ -67,6 +68,7 @@ constexpr int kBM = kWaves * kQW;        // queries per workgroup
 constexpr uint32_t kTile = kBN * kD * 2;  // bytes of one K or V tile
 constexpr uint32_t kList = 4 * kTile;     // key-list ring: 3 slots of one tile's 64 entries
 constexpr uint32_t kLds = kList + 3 * kBN * 4;
+constexpr float kNoKey = -3.0e38f;        // reference max before any key
 constexpr float kLazy = 8.0f;             // log2 headroom before the reference max moves
 
 struct Params {
@@ -81,7 +83,14 @@ struct Params {
     float c;                         // softmax scale * log2(e)
     State *o_st;                     // amax of the output folded here, or null
     uint32_t o_shift;                // 16: folded as fp32 magnitude bits, 0: as bf16 bits
+    int full, splits;                // query tiles [0, full) whole, the others in `splits` key ranges
+    float *part;                     // the ranges' partials (kPart floats each)
 };
+
+// One key range of one query tile: the waves' O accumulators unscaled, 1 KB per store instruction
+// ([wave][qb][d][lane] f32x4), then each query's reference max (log2) and sum ([2][wave][qb][16]).
+constexpr int kPartO = kBM * kD;
+constexpr int kPart = kPartO + 2 * kBM;
 
 #define ASMV asm volatile
 
@@ -150,17 +159,28 @@ __device__ __forceinline__ float max_over_groups(float m)
 // entries reach LDS the way K and V do (wave 0 loads a tile's 64 entries two tiles ahead into a
 // ring of three slots), so the loop holds no global load whose wait would also wait for the
 // K and V loads of the next tile.
-template <bool LIST> __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const Params p)
+// SPLIT: a launch with key ranges (an instantiation of its own: the loop from a variable first tile
+// ran the list form up to 4 % slower).
+template <bool LIST, bool SPLIT> __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(const Params p)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[kLds];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t cq = lane & 15u, g = lane >> 4;
 
-    // workgroup -> (batch, head, query tile), consecutive query tiles of a head on one XCD
-    const int nwg = gridDim.x, w = blockIdx.x;
-    const int per = nwg >> 3, rem = nwg & 7, xcd = w & 7, slot = w >> 3;
-    const int L = xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
+    // workgroup -> (batch, head, query tile), consecutive query tiles of a head on one XCD; from
+    // `full` on, workgroup full + i is key range i % splits of tile full + i / splits (8 ranges or a
+    // multiple: a range of the head's tiles stays on one XCD)
+    const int nwg = SPLIT ? p.full : gridDim.x, w = blockIdx.x;
+    const bool split = SPLIT && w >= nwg;
+    int L, range = 0;
+    if (!split) {
+        const int per = nwg >> 3, rem = nwg & 7, xcd = w & 7, slot = w >> 3;
+        L = xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
+    } else {
+        L = nwg + (w - nwg) / p.splits;
+        range = (w - nwg) % p.splits;
+    }
     const int qt = L % p.q_tiles, bh = L / p.q_tiles;
     const int h = bh % p.heads, b = bh / p.heads;
 
@@ -171,7 +191,12 @@ template <bool LIST> __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(c
         if (p.key_idx && int64_t(nk) > p.idx_bs) nk = int(p.idx_bs);
     }
     nk = __builtin_amdgcn_readfirstlane(nk);
-    const int ntiles = (nk + kBN - 1) / kBN;
+    int t0 = 0, ntiles = (nk + kBN - 1) / kBN;   // this workgroup's key tiles: t0 .. ntiles - 1
+    if (split) {
+        const int len = (ntiles + p.splits - 1) / p.splits;
+        t0 = range * len;
+        ntiles = ntiles < t0 + len ? ntiles : t0 + len;
+    }
 
     // buffer resources of this (batch, head)'s K and V: rows of 256 bytes at the row stride; the
     // range ends with the last key row
@@ -260,14 +285,14 @@ template <bool LIST> __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(c
         }
     };
 
-    if (ntiles > 0) {
+    if (ntiles > t0) {
         if (LIST) {
-            list_dtl(0);
-            if (ntiles > 1) list_dtl(1);
+            list_dtl(t0);
+            if (ntiles > t0 + 1) list_dtl(t0 + 1);
             ASMV("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
         }
-        issue_tile(0);
+        issue_tile(t0);
     }
 
     // Q fragments: lane (cq, g) holds dims 32 pp + 8 g .. +7 of query 16 qb + cq of the wave's 32
@@ -288,7 +313,8 @@ template <bool LIST> __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(c
 #pragma unroll
     for (int d = 0; d < 8; ++d)
         o[d][0] = o[d][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float mref[2] = {-__builtin_inff(), -__builtin_inff()};
+    // below every score, and finite: keys whose scores are all -inf get probabilities 0
+    float mref[2] = {kNoKey, kNoKey};
     float lsum[2] = {0.f, 0.f};
     const float c = p.c;
 
@@ -303,7 +329,7 @@ template <bool LIST> __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(c
 #pragma unroll
     for (int pp = 0; pp < 4; ++pp) ka[pp] = kfrag + (((4u * pp + g) ^ cq) << 4);
     const uint32_t va_e = vfrag + (g & 1u) * 128u, va_o = vfrag - (g & 1u) * 128u;
-    for (int t = 0; t < ntiles; ++t) {
+    for (int t = t0; t < ntiles; ++t) {
         ASMV("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (t + 1 < ntiles) issue_tile(t + 1);
@@ -393,6 +419,23 @@ template <bool LIST> __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(c
         }
     }
 
+    if (split) {
+        float *P = p.part + size_t(w - nwg) * kPart;
+        f32x4 *po = (f32x4 *)P + wave * 1024u + lane;
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+#pragma unroll
+            for (int d = 0; d < 8; ++d) po[(qb * 8 + d) * 64] = o[d][qb];
+            float l = lsum[qb];
+            l += __shfl_xor(l, 16, 64);
+            l += __shfl_xor(l, 32, 64);
+            if (g == 0) {
+                P[kPartO + wave * 32u + qb * 16u + cq] = mref[qb];
+                P[kPartO + kBM + wave * 32u + qb * 16u + cq] = l;
+            }
+        }
+        return;
+    }
     // epilogue: O / l, rounded to bf16; lane (cq, g) holds dims 16 d + 4 g .. +3 of query 16 qb + cq
     uint32_t amax = 0;
 #pragma unroll
@@ -432,6 +475,58 @@ template <bool LIST> __global__ __launch_bounds__(kThreads, 1) void k_attn_fwd(c
     }
 }
 
+// The split tiles' outputs: the key ranges' partials of each query moved to the largest of their
+// reference maxima and added in range order (deterministic), divided by the sum, rounded and stored as
+// the kernel's own epilogue does, with the amax folded.  A range without keys has max kNoKey, sum 0
+// and O 0.  One wave per (tile, wave of the tile, query block, 2 of the 8 dim blocks).
+__global__ __launch_bounds__(256) void k_attn_combine(const Params p)
+{
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, cq = lane & 15u, g = lane >> 4;
+    const int tile = int(blockIdx.x / 24u);
+    const uint32_t u = (blockIdx.x % 24u) * 4u + (tid >> 6);
+    const uint32_t wave = u >> 3, qb = (u >> 2) & 1u, dp = u & 3u;
+    const int L = p.full + tile;
+    const int qt = L % p.q_tiles, bh = L / p.q_tiles;
+    const int h = bh % p.heads, b = bh / p.heads;
+    const float *P = p.part + size_t(tile) * size_t(p.splits) * kPart;
+    const uint32_t ml = kPartO + wave * 32u + qb * 16u + cq;
+    float m = kNoKey;
+    for (int s = 0; s < p.splits; ++s) m = __builtin_elementwise_maximum(m, P[size_t(s) * kPart + ml]);
+    f32x4 o0 = f32x4{0.f, 0.f, 0.f, 0.f}, o1 = o0;
+    float l = 0.f;
+    for (int s = 0; s < p.splits; ++s) {
+        const float *Ps = P + size_t(s) * kPart;
+        const float a = __builtin_amdgcn_exp2f(Ps[ml] - m);
+        const f32x4 *po = (const f32x4 *)Ps + wave * 1024u + (qb * 8u + 2u * dp) * 64u + lane;
+        l = __builtin_fmaf(a, Ps[ml + kBM], l);
+        o0 += a * po[0];
+        o1 += a * po[64];
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const int row = qt * kBM + int(wave) * kQW + int(qb) * 16 + int(cq);
+    uint32_t amax = 0;
+    if (row < p.n_q) {
+        uint16_t *orow = p.out + int64_t(b) * p.o_bs + int64_t(row) * p.o_rs + int64_t(h) * kD + 4 * g + 32 * dp;
+        const u32x2 w0 = u32x2{pk_bf16(o0[0] * inv, o0[1] * inv), pk_bf16(o0[2] * inv, o0[3] * inv)};
+        const u32x2 w1 = u32x2{pk_bf16(o1[0] * inv, o1[1] * inv), pk_bf16(o1[2] * inv, o1[3] * inv)};
+        *(u32x2 *)orow = w0;
+        *(u32x2 *)(orow + 16) = w1;
+        const uint32_t v[4] = {w0.x & 0x7FFF7FFFu, w0.y & 0x7FFF7FFFu, w1.x & 0x7FFF7FFFu, w1.y & 0x7FFF7FFFu};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) amax = max(amax, max(v[i] & 0xFFFFu, v[i] >> 16));
+    }
+    if (p.o_st) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, off, 64));
+        __shared__ uint32_t wmax[4];
+        if (lane == 0) wmax[tid >> 6] = amax;
+        __syncthreads();
+        if (tid == 0)
+            __hip_atomic_fetch_max(&p.o_st->amax_acc, max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])) << p.o_shift,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 // The o projection's state after the attention: amax of the output (bf16, or as fp32 values),
 // its scale for smax and the tables.
 __global__ __launch_bounds__(256) void k_attn_amax_settle(State *__restrict__ st, int dtype, float smax)
@@ -440,13 +535,64 @@ __global__ __launch_bounds__(256) void k_attn_amax_settle(State *__restrict__ st
     settle_amax(st, dtype, smax, lds);
 }
 
+static int cu_count()
+{
+    static int cus[64] = {0};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (cus[dev] == 0) {
+        int c = 0;
+        if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0) c = 256;
+        cus[dev] = c;
+    }
+    return cus[dev];
+}
+
+// The last wave of query tiles (one workgroup fills a CU) in key ranges, where that ends sooner: the
+// tiles past the last whole wave as `splits` ranges each, at least 2 key tiles a range, at most 3 waves
+// of ranges (150 MB of partials on 256 CUs).  A workgroup takes about 15 us and 2.6 us per 64-key tile;
+// a range's partial costs 0.1 us of the chip to write and add up, and the adding kernel 5 us.  The
+// 1.3B 480P self-attention's 1032 tiles are 4 waves and 8 tiles, which ran a fifth wave alone: 6.65 ->
+// 5.25 ms (990 -> 1255 TFLOP/s).  From 8 waves up the CUs' tile boundaries have drifted apart and the
+// tail fills in by itself (14.4 waves: 1 % slower split).
+struct Plan {
+    int full, splits;
+    int64_t parts(int64_t tiles) const { return splits > 1 ? (tiles - full) * splits : 0; }
+};
+static Plan plan_split(int64_t tiles, int64_t n_kv)
+{
+    const int64_t cus = cu_count(), tail = tiles % cus, nt = (n_kv + kBN - 1) / kBN;
+    Plan best{int(tiles), 1};
+    if (tail == 0 || tiles >= 8 * cus) return best;
+    auto wave_us = [](int64_t key_tiles) { return 15.0 + 2.6 * double(key_tiles); };
+    double least = 0.9 * wave_us(nt);
+    for (int64_t sp = 2; sp <= 32 && nt >= 2 * sp && tail * sp <= 3 * cus; ++sp) {
+        const double us = double((tail * sp + cus - 1) / cus) * wave_us((nt + sp - 1) / sp) + 5.0 + 0.1 * double(tail * sp);
+        if (us < least) {
+            least = us;
+            best = Plan{int(tiles - tail), int(sp)};
+        }
+    }
+    return best;
+}
+
 }  // namespace attn
 
-extern "C" int hif8_attention_fwd(const uint16_t *q, const uint16_t *k, const uint16_t *v, uint16_t *out,
-                                  int64_t batch, int64_t n_q, int64_t n_kv, int64_t heads, int64_t head_dim,
-                                  const int64_t *row_strides, const int64_t *batch_strides, const int32_t *key_idx,
-                                  int64_t idx_batch_stride, const int32_t *key_count, float softmax_scale,
-                                  void *out_state, int out_state_dtype, float scale_max, hif8_stream_t stream)
+extern "C" int64_t hif8_attention_workspace_bytes(int64_t batch, int64_t n_q, int64_t n_kv, int64_t heads)
+{
+    using namespace attn;
+    if (batch <= 0 || n_q <= 0 || n_kv <= 0 || heads <= 0) return 0;
+    const int64_t tiles = batch * heads * ((n_q + kBM - 1) / kBM);
+    if (tiles >= (int64_t(1) << 31)) return 0;
+    return plan_split(tiles, n_kv).parts(tiles) * kPart * 4;
+}
+
+extern "C" int hif8_attention_fwd_split(const uint16_t *q, const uint16_t *k, const uint16_t *v, uint16_t *out,
+                                        int64_t batch, int64_t n_q, int64_t n_kv, int64_t heads, int64_t head_dim,
+                                        const int64_t *row_strides, const int64_t *batch_strides,
+                                        const int32_t *key_idx, int64_t idx_batch_stride, const int32_t *key_count,
+                                        float softmax_scale, void *out_state, int out_state_dtype, float scale_max,
+                                        void *workspace, int64_t workspace_bytes, hif8_stream_t stream)
 {
     using namespace attn;
     if (!q || !k || !v || !out || !row_strides || !batch_strides) return HIF8_ERR_ARG;
@@ -494,15 +640,43 @@ extern "C" int hif8_attention_fwd(const uint16_t *q, const uint16_t *k, const ui
     p.c = float(double(softmax_scale) * 1.4426950408889634);
     p.o_st = (State *)out_state;
     p.o_shift = out_state_dtype == kBF16F32 ? 16u : 0u;
+    const int64_t tiles = batch * heads * q_tiles;
+    Plan plan{int(tiles), 1};
+    if (workspace) {
+        plan = plan_split(tiles, n_kv);
+        if (workspace_bytes < plan.parts(tiles) * kPart * 4) return HIF8_ERR_ARG;
+        if ((uintptr_t)workspace & 15u) return HIF8_ERR_ALIGN;
+    }
+    p.full = plan.full;
+    p.splits = plan.splits;
+    p.part = (float *)workspace;
     hipStream_t s = (hipStream_t)stream;
-    if (key_idx)
-        hipLaunchKernelGGL(k_attn_fwd<true>, dim3(unsigned(batch * heads * q_tiles)), dim3(kThreads), 0, s, p);
+    const unsigned wgs = unsigned(plan.full + plan.parts(tiles));
+    if (key_idx && plan.splits > 1)
+        hipLaunchKernelGGL((k_attn_fwd<true, true>), dim3(wgs), dim3(kThreads), 0, s, p);
+    else if (key_idx)
+        hipLaunchKernelGGL((k_attn_fwd<true, false>), dim3(wgs), dim3(kThreads), 0, s, p);
+    else if (plan.splits > 1)
+        hipLaunchKernelGGL((k_attn_fwd<false, true>), dim3(wgs), dim3(kThreads), 0, s, p);
     else
-        hipLaunchKernelGGL(k_attn_fwd<false>, dim3(unsigned(batch * heads * q_tiles)), dim3(kThreads), 0, s, p);
+        hipLaunchKernelGGL((k_attn_fwd<false, false>), dim3(wgs), dim3(kThreads), 0, s, p);
+    if (plan.splits > 1)
+        hipLaunchKernelGGL(k_attn_combine, dim3(unsigned(tiles - plan.full) * 24u), dim3(256), 0, s, p);
     if (out_state)
         hipLaunchKernelGGL(k_attn_amax_settle, dim3(1), dim3(256), 0, s, (State *)out_state,
                            out_state_dtype == kBF16F32 ? kF32 : kBF16, scale_max);
     return hipGetLastError() == hipSuccess ? HIF8_OK : HIF8_ERR_HIP;
+}
+
+extern "C" int hif8_attention_fwd(const uint16_t *q, const uint16_t *k, const uint16_t *v, uint16_t *out,
+                                  int64_t batch, int64_t n_q, int64_t n_kv, int64_t heads, int64_t head_dim,
+                                  const int64_t *row_strides, const int64_t *batch_strides, const int32_t *key_idx,
+                                  int64_t idx_batch_stride, const int32_t *key_count, float softmax_scale,
+                                  void *out_state, int out_state_dtype, float scale_max, hif8_stream_t stream)
+{
+    return hif8_attention_fwd_split(q, k, v, out, batch, n_q, n_kv, heads, head_dim, row_strides, batch_strides,
+                                    key_idx, idx_batch_stride, key_count, softmax_scale, out_state, out_state_dtype,
+                                    scale_max, nullptr, 0, stream);
 }
 
 }  // namespace hif8

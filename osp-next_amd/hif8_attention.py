@@ -122,8 +122,9 @@ def attention_fwd(q: Tensor, k: Tensor, v: Tensor, key_idx: Optional[Tensor] = N
     key_idx[b, :key_count[b]], as ``key_list`` gives them).  ``softmax_scale`` defaults to
     1/sqrt(128), SDPA's.  With ``o_state``, the amax of out is left in it with the scale rule
     for ``scale_max`` (as fp32 values with ``o_as_f32``, the self-attention's o input), as
-    ``absmax_scale(out, scale_max, o_state, o_as_f32)`` would leave it.  Inference only (no
-    backward)."""
+    ``absmax_scale(out, scale_max, o_state, o_as_f32)`` would leave it.  A last wave of workgroups that
+    would leave CUs idle runs as key ranges (a transient workspace of
+    ``hif8_attention_workspace_bytes``).  Inference only (no backward)."""
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
         raise RuntimeError("attention_fwd has no backward; use attention_with_mask under autograd")
     if not attention_fwd_ok(q, k, v):
@@ -152,8 +153,11 @@ def attention_fwd(q: Tensor, k: Tensor, v: Tensor, key_idx: Optional[Tensor] = N
     scale = 1.0 / math.sqrt(D) if softmax_scale is None else float(softmax_scale)
     st_ptr = o_state.ptr if o_state is not None else 0
     st_dtype = _lib.DTYPE_BF16_AS_F32 if o_as_f32 else _lib.DTYPE_BF16
-    _lib.check(_lib.load().hif8_attention_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, Nq, Nkv,
-                                              H, D, rs, bs, idx_ptr, idx_bs, cnt_ptr, scale, st_ptr, st_dtype,
-                                              float(scale_max), _lib.stream_ptr(q.device)),
-               "hif8_attention_fwd")
+    L = _lib.load()
+    nbytes = int(L.hif8_attention_workspace_bytes(B, Nq, Nkv, H))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes > 0 else None
+    _lib.check(L.hif8_attention_fwd_split(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, Nq, Nkv, H, D, rs,
+                                          bs, idx_ptr, idx_bs, cnt_ptr, scale, st_ptr, st_dtype, float(scale_max),
+                                          ws.data_ptr() if ws is not None else None, nbytes,
+                                          _lib.stream_ptr(q.device)), "hif8_attention_fwd_split")
     return out
