@@ -473,6 +473,11 @@ static int launch(const uint16_t *x, const uint8_t *w_codes, const Groups &g, co
     const int tiles_n = int((N + dtl::kTile - 1) / dtl::kTile);
     const int64_t tiles = int64_t(tiles_m) * tiles_n;
     if (tiles >= (int64_t(1) << 31)) return HIF8_ERR_SHAPE;
+    if (const int tile = small_linear_tile(M, N, K)) {
+        const int rc = launch_linear_small(tile, x, w_codes, g, bias, M, N, K, y_st, stream);
+        if (rc != HIF8_OK) return rc;
+        return y_st ? launch_gelu_stat_settle(y_st, y_smax, stream) : HIF8_OK;
+    }
     if (y_st)
         hipLaunchKernelGGL(dtl::k_linear_dtl<1>, dim3(unsigned(tiles)), dim3(dtl::kThreads), 0, s, x, w_codes, g, bias,
                            int(M), int(N), int(K), tiles_m, tiles_n, y_st);
