@@ -28,19 +28,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // ---------------------------------------------------------------- kernels
 
-__global__ void k_state_init(State *st)
-{
-    if (threadIdx.x == 0) {
-        st->counter = 0;
-        st->amax_acc = 0;
-        st->amax_bits = 0;
-        st->scale = 0.0f;
-        st->fast = 0;
-        st->dtype = 0;
-        st->finite = 0;
-        st->pending = 0;
-    }
-}
+__global__ void k_state_init(State *st) { init_state(st); }
 
 __global__ __launch_bounds__(256) void k_set_scale(State *st, int dtype, float s)
 {

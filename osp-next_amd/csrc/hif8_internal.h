@@ -16,6 +16,8 @@ constexpr int kSemTorch = HIF8_SEM_TORCH;
 // Entries of the GELU quantisation pass's table of x_q over y (hif8_codec.hip, k_gelu_quant).
 constexpr uint32_t kGqCap = 5248;
 
+constexpr int kFoldSlots = 32;
+
 // Per-tensor quantisation state (device memory, hif8_state_size() bytes).
 struct alignas(256) State {
     uint32_t counter;      // workgroups finished in the running amax pass (reset by the last)
@@ -34,6 +36,11 @@ struct alignas(256) State {
     // top (the last entry).
     uint32_t gq[4];
     uint32_t gq_tab[kGqCap];
+    // First level of an amax pass's fold (hif8_state_dev.h): the maximum and the count of one group of
+    // workgroups each, a cache line apart; zero between passes.
+    struct alignas(128) Fold {
+        uint32_t max, count;
+    } fold[kFoldSlots];
 };
 
 static_assert(sizeof(State) % 256 == 0, "state size");

@@ -47,8 +47,11 @@ constexpr int kTPB = 256;
 constexpr int kWaves = kTPB / 64;
 constexpr int kMaxChunks = 16;   // 16-B chunks per lane: dim <= 16 * 64 * 8 = 8192
 constexpr int kWgPerCu = 3;     // pass 1 (157 VGPRs at dim 5120: 3 wavefronts per SIMD)
-constexpr int kExtWgPerCu = 2;  // pass 1 from per-column extremes (k_modln_amax_ext)
 constexpr int kQdqWgPerCu = 2;  // pass 2 (2 workgroups per CU streamed 1.2-1.4 % faster than 3 at 14B 720P)
+// Pass 1 from per-column extremes (k_modln_amax_ext) keeps one row per wavefront in flight: 2
+// workgroups per CU are best for wide rows (5120: 137 us at 75600 rows, 145 with 4), narrow ones (up to
+// 2048) want more of them in flight (1536, 32760 rows: 34 us with 2, 26 with 4).
+constexpr int ext_wg_per_cu(int nch) { return nch <= 4 ? 4 : 2; }
 
 // Sum over the wavefront, returned to every lane: DPP steps within each row of 16 lanes
 // (quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror, row_mirror), then the four row sums.
@@ -442,7 +445,7 @@ __global__ __launch_bounds__(kTPB) void k_modln_amax(const uint16_t *__restrict_
 // variance, where (x - mean) * 0 can be NaN) are not folded: a wavefront that meets one
 // re-reads all its rows after the loop and takes every y through the full chain, as the
 // per-element pass does, so NaN rows give the same NaN bits.  One row in registers at a time:
-// 151 VGPRs, 3 wavefronts per SIMD; 2 workgroups per CU stream x faster than 3 here.
+// 151 VGPRs at dim 5120, 3 wavefronts per SIMD.
 template <int NCH>
 __global__ __launch_bounds__(kTPB) __attribute__((amdgpu_waves_per_eu(3))) void k_modln_amax_ext(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ shift, const uint16_t *__restrict__ scale,
@@ -760,7 +763,7 @@ static void launch_amax(bool modl, int grid, hipStream_t s, const uint16_t *x, c
 {
     if constexpr (NCH <= 10) {
         if (modl) {
-            const int g = grid_for_rows(rows, kExtWgPerCu);
+            const int g = grid_for_rows(rows, ext_wg_per_cu(NCH));
             hipLaunchKernelGGL((k_modln_amax_ext<NCH>), dim3(g), dim3(kTPB), size_t(8 * dim), s, x, shift, scale,
                                rows, dim, eps, stats, st, smax);
             return;
@@ -855,19 +858,7 @@ static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
 // Clears the counters and scalars of the state in the workspace (the previous call leaves them
 // zero unless it was interrupted); a fill kernel, so a captured graph holds no memset node.
-__global__ void k_scratch_state_clear(State *st)
-{
-    if (threadIdx.x == 0) {
-        st->counter = 0;
-        st->amax_acc = 0;
-        st->amax_bits = 0;
-        st->scale = 0.0f;
-        st->fast = 0;
-        st->dtype = 0;
-        st->finite = 0;
-        st->pending = 0;
-    }
-}
+__global__ void k_scratch_state_clear(State *st) { init_state(st); }
 
 static std::mutex g_scratch_mu;
 static uint8_t *g_scratch_dev[64];

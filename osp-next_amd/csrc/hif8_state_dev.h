@@ -69,27 +69,69 @@ __device__ __forceinline__ float write_amax_state(State *st, uint32_t a, int dty
     return s;
 }
 
+// Zero the words an amax pass counts on, and the scalars of st (one workgroup of at least 64 threads).
+__device__ __forceinline__ void init_state(State *st)
+{
+    const uint32_t tid = threadIdx.x;
+    if (tid == 0) {
+        st->counter = 0;
+        st->amax_acc = 0;
+        st->amax_bits = 0;
+        st->scale = 0.0f;
+        st->fast = 0;
+        st->dtype = 0;
+        st->finite = 0;
+        st->pending = 0;
+    }
+    if (tid < uint32_t(kFoldSlots)) {
+        st->fold[tid].max = 0;
+        st->fold[tid].count = 0;
+    }
+}
+
+// m folded into *max and this participant counted in *count; true for the last of n, with m then the
+// maximum of all of them and both words zero again.  The atomics are relaxed: the maximum's is waited
+// for (its old value is used) before the count's is issued, so the participant that counts last finds
+// every maximum, and nothing else is passed between workgroups.
+__device__ __forceinline__ bool fold_last(uint32_t *max, uint32_t *count, uint32_t n, uint32_t &m)
+{
+    const uint32_t old = __hip_atomic_fetch_max(max, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::"v"(old) : "memory");
+    if (__hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != n - 1) return false;
+    m = __hip_atomic_exchange(max, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
 // Fold one workgroup's amax (magnitude bits; NaN above every finite value) into st;
-// the last of `nwg` workgroups resets the accumulators and writes amax, scale, flags
+// the last of the grid's `nwg` workgroups resets the accumulators and writes amax, scale, flags
 // and the tables.  Called by all 256 threads of the workgroup with `m` already reduced
 // over it (only thread 0's value is used); `lds` is two words of LDS scratch.
+// Two levels: workgroups count into kFoldSlots groups, the last of each into the root.  Atomics on one
+// address take turns, about 25 ns a workgroup on one pair of words (and twice that with an
+// acquire-release count, which wrote back and invalidated the XCD's L2 each time).  One address and
+// acquire-release -> two levels: the 2048 workgroups of the q/k norm + rope amax pass on [32760, 1536]
+// 109 -> 30 us, the modulated norm's 1024 there 46 -> 26, 500 workgroups on [2000, 1536] 18.5 -> 7.5, the
+// amax pass of [4096, 5120] (256 workgroups) 13.4 -> 9.7.
 __device__ __forceinline__ void fold_amax(State *st, uint32_t m, uint32_t nwg, int dtype, float smax,
                                           uint32_t *lds)
 {
     const uint32_t tid = threadIdx.x;
     if (tid == 0) {
-        __hip_atomic_fetch_max(&st->amax_acc, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t prev = __hip_atomic_fetch_add(&st->counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        lds[0] = (prev == nwg - 1) ? 1u : 0u;
+        bool last = true;
+        uint32_t roots = nwg;
+        if (nwg >= 2u * kFoldSlots) {
+            const uint32_t slot = blockIdx.x % kFoldSlots;
+            roots = kFoldSlots;
+            last = fold_last(&st->fold[slot].max, &st->fold[slot].count,
+                             nwg / kFoldSlots + (slot < nwg % kFoldSlots ? 1u : 0u), m);
+        }
+        if (last) last = fold_last(&st->amax_acc, &st->counter, roots, m);
+        lds[0] = last ? 1u : 0u;
+        if (last) lds[1] = f2u(write_amax_state(st, m, dtype, smax));
     }
     __syncthreads();
     if (!lds[0]) return;
-    if (tid == 0) {
-        const uint32_t a = __hip_atomic_exchange(&st->amax_acc, 0u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&st->counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        lds[1] = f2u(write_amax_state(st, a, dtype, smax));
-    }
-    __syncthreads();
     fill_luts(st, u2f(lds[1]), tid);
 }
 
