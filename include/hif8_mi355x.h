@@ -92,6 +92,18 @@ int hif8_absmax_scale(const void *x, int dtype, int64_t n, float scale_max, void
  * for callers that carry their own scale. */
 int hif8_set_scale(void *state, int dtype, float scale, hif8_stream_t stream);
 
+/* hif8_state_init, hif8_absmax_scale and the quantisation of x in two launches: the amax pass leaves its
+ * workgroups' maxima in state, which need not be initialised, and the quantisation pass reduces them
+ * and settles state as hif8_absmax_scale would (the reference's _quant, hif8_linear.py:42-50).
+ * out_kind HIF8_OUT_CODES: hif8_encode's codes (semantics HIF8_SEM_NPU); HIF8_OUT_SAME: hif8_fake_quant's
+ * x_q; HIF8_OUT_BF16: hif8_fake_quant_to_bf16's; the same bytes as those entry points give.  x and out
+ * 16-byte aligned, n > 0. */
+#define HIF8_OUT_CODES 0
+#define HIF8_OUT_SAME 1
+#define HIF8_OUT_BF16 3
+int hif8_quantize(const void *x, int dtype, int64_t n, float scale_max, void *state, void *out, int out_kind,
+                  int semantics, hif8_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * Encode: HiF8 codes of qdq(x * scale), NPU semantics (hif8_linear.py:47-48 with
  * QTensor.py:94-128 -> hif8_quant_op.h:88-151).  codes: n bytes.

@@ -20,6 +20,7 @@ DTYPE_BF16, DTYPE_F32, DTYPE_BF16_AS_F32 = 0, 1, 2
 SEM_NPU, SEM_TORCH, SEM_TORCH_BF16, SEM_TORCH_F16 = 0, 1, 2, 3
 # formats of a quantised activation held by the Python layer: bf16 x_q, or its 8-bit codes
 A_BF16, A_CODES = 0, 1
+OUT_CODES, OUT_SAME, OUT_BF16 = 0, 1, 3    # HIF8_OUT_*: what hif8_quantize writes
 
 # Every symbol the header declares, with (restype, argtypes).
 _p, _i, _i64, _f, _sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_size_t
@@ -30,6 +31,7 @@ SIGNATURES = {
     "hif8_state_read": (_i, [_p, ctypes.POINTER(ctypes.c_uint32), ctypes.POINTER(ctypes.c_float), _p]),
     "hif8_absmax_scale": (_i, [_p, _i, _i64, _f, _p, _p]),
     "hif8_set_scale": (_i, [_p, _i, _f, _p]),
+    "hif8_quantize": (_i, [_p, _i, _i64, _f, _p, _p, _i, _i, _p]),
     "hif8_encode": (_i, [_p, _i, _i64, _p, _p, _p]),
     "hif8_fake_quant": (_i, [_p, _i, _i64, _p, _p, _i, _p]),
     "hif8_fake_quant_to_bf16": (_i, [_p, _i, _i64, _p, _p, _i, _p]),
@@ -110,7 +112,9 @@ def check(status: int, what: str) -> None:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle, without building a Stream object (four or more times a linear)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(t: torch.Tensor) -> int:
@@ -125,8 +129,19 @@ def dtype_code(dt: torch.dtype) -> int:
     raise TypeError(f"HiF8 kernels take bfloat16 or float32 tensors, got {dt}")
 
 
+_state_size = 0
+
+
 def state_size() -> int:
-    return int(load().hif8_state_size())
+    global _state_size
+    if _state_size == 0:
+        _state_size = int(load().hif8_state_size())
+    return _state_size
+
+
+def unset_state(device: torch.device) -> torch.Tensor:
+    """A state buffer for hif8_quantize, which needs no initialised one."""
+    return torch.empty(state_size(), dtype=torch.uint8, device=device)
 
 
 def new_state(device: torch.device) -> torch.Tensor:

@@ -46,6 +46,12 @@ __global__ __launch_bounds__(256) void k_set_scale(State *st, int dtype, float s
 
 constexpr int kTPB = 256;
 
+// The workgroup maxima of an amax pass without a fold (at most kMaxParts of them), in the words that
+// later hold the GELU quantisation's table.
+constexpr int kMaxParts = kTPB;
+static_assert(uint32_t(kMaxParts) <= kGqCap, "one word per workgroup");
+__device__ __forceinline__ uint32_t *amax_parts(State *st) { return st->gq_tab; }
+
 // Streaming access: the codec reads each input element once, so its global loads carry
 // the non-temporal hint (measured on the 774 MB 14B activation: amax 4.98 -> 6.5 TB/s).
 // Code output (1 B/element) is stored the same way; bf16/fp32 qdq output is stored
@@ -61,7 +67,11 @@ template <typename T> __device__ __forceinline__ void st_stream(T *p, const T &v
 
 // One pass of |x| max.  Magnitude bit patterns order like the values and put
 // NaN above Inf, so an unsigned max propagates NaN as torch's amax does.
-template <int DT>
+// PART: each workgroup leaves its maximum in the state's scratch words (amax_parts) for the k_quant that
+// follows, which reduces them itself: no atomics, and no state that has to be initialised.  The three
+// launches init, amax, quantise -> these two (us): 98304 bf16 elements 10.7 -> 6.8, [512, 5120] 11.8 ->
+// 8.0, [4096, 5120] 29 -> 25, [75600, 5120] 370 -> 368.
+template <int DT, bool PART = false>
 __global__ __launch_bounds__(kTPB) void k_absmax(const void *__restrict__ xv, int64_t n,
                                                   State *__restrict__ st, float smax)
 {
@@ -133,6 +143,10 @@ __global__ __launch_bounds__(kTPB) void k_absmax(const void *__restrict__ xv, in
     __syncthreads();
     m = max(max(red[0], red[1]), max(red[2], red[3]));
     // bf16 held as fp32: the fp32 magnitude bits of the same value (NaN stays above Inf)
+    if (PART) {
+        if (tid == 0) amax_parts(st)[blockIdx.x] = DT == kBF16F32 ? m << 16 : m;
+        return;
+    }
     if (DT == kBF16F32) fold_amax(st, m << 16, gridDim.x, kF32, smax, red + kTPB / 64);
     else fold_amax(st, m, gridDim.x, DT, smax, red + kTPB / 64);
 }
@@ -161,10 +175,13 @@ __device__ __forceinline__ void scalar_elem(const void *xv, void *outv, int64_t 
 // span > 0: workgroup b quantises the span * TPB consecutive 16-element groups from
 // b * span * TPB on (the grid covers the tensor once, in dispatch order, so the groups in flight
 // at any time lie in one moving window of memory); span 0: a grid-stride loop.
+// parts > 0: the amax, scale and decode tables come from the parts workgroup maxima that k_absmax<DT, true>
+// left in st, reduced by every workgroup for itself; workgroup 0 writes them into st as an amax pass
+// settles it, counters included (st may have been uninitialised).
 template <int DT, int MODE, int TPB = kTPB>
 __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int64_t n,
-                                                 const State *__restrict__ st, void *__restrict__ outv,
-                                                 int sem, int use_state, int span)
+                                                 State *st, void *__restrict__ outv,
+                                                 int sem, int use_state, int span, int parts, float smax)
 {
     __shared__ __attribute__((aligned(16))) uint8_t lds[kLdsBytes];
     const int tid = threadIdx.x;
@@ -193,13 +210,40 @@ __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int6
             if (c < nchunk) pre[j] = ld_stream(&xq[c]);
         }
     }
-    float s = use_state ? st->scale : 1.0f;
-    bool fast = use_state ? (st->fast != 0) : true;
-    // NaN inputs map to the +Inf entry of the table; unless an amax pass proved
-    // the tensor finite, each 16-element group is checked and patched to kNanCode.
-    const bool nan_guard = use_state ? (st->finite == 0) : true;
+    float s;
+    bool fast, nan_guard;
+    if (MODE != 2 && parts > 0) {
+        uint32_t m = tid < parts ? amax_parts(st)[tid] : 0u;
+        for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
+        __shared__ uint32_t red[TPB / 64];
+        if ((tid & 63) == 0) red[tid >> 6] = m;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < TPB / 64; ++w) m = max(m, red[w]);
+        constexpr int kStateDt = DT == kBF16 ? kBF16 : kF32;
+        s = scale_from_amax(m, kStateDt, smax, fast);
+        nan_guard = !fast;
+        if (blockIdx.x == 0) {
+            init_state(st);
+            __syncthreads();
+            if (tid == 0) write_amax_state(st, m, kStateDt, smax);
+            if (tid < 256) fill_luts(st, s, uint32_t(tid));
+        }
+    } else {
+        s = use_state ? st->scale : 1.0f;
+        fast = use_state ? (st->fast != 0) : true;
+        // NaN inputs map to the +Inf entry of the table; unless an amax pass proved
+        // the tensor finite, each 16-element group is checked and patched to kNanCode.
+        nan_guard = use_state ? (st->finite == 0) : true;
+    }
     // decode tables for this scale
-    if (tid < 256) {
+    if (MODE != 2 && parts > 0) {
+        if (tid < 256) {
+            const float y = u2f(decode_bits(uint32_t(tid))) / s;
+            ((float *)(lds + kLdsLutF32))[tid] = y;
+            ((uint16_t *)(lds + kLdsLutBf16))[tid] = uint16_t(f2bf(y));
+        }
+    } else if (tid < 256) {
         uint32_t c = uint32_t(tid);
         float y;
         if (use_state) y = st->lut_f32[c];
@@ -903,8 +947,8 @@ template <int DT, int MODE> static int resident_wgs()
 }
 
 template <int DT, int MODE>
-static void launch_k_quant(const void *x, int64_t n, const State *st, void *out, int sem, int use_state, int wg_per_cu,
-                           hipStream_t s)
+static void launch_k_quant(const void *x, int64_t n, State *st, void *out, int sem, int use_state, int wg_per_cu,
+                           hipStream_t s, int parts = 0, float smax = 0.0f)
 {
     const int64_t ngrp = (n + 15) / 16;
     int grid, span = 0;
@@ -917,7 +961,8 @@ static void launch_k_quant(const void *x, int64_t n, const State *st, void *out,
         const int fit = resident_wgs<DT, MODE>();
         grid = grid_for(ngrp, cu_count() * (wg_per_cu < fit ? wg_per_cu : fit));
     }
-    hipLaunchKernelGGL((k_quant<DT, MODE>), dim3(grid), dim3(kTPB), 0, s, x, n, st, out, sem, use_state, span);
+    hipLaunchKernelGGL((k_quant<DT, MODE>), dim3(grid), dim3(kTPB), 0, s, x, n, st, out, sem, use_state, span,
+                       parts, smax);
 }
 
 // The GELU route: the prep kernel, then spans of HIF8_GELU_SPAN x 256 groups per workgroup
@@ -1010,7 +1055,8 @@ int hif8_set_scale(void *state, int dtype, float scale, hif8_stream_t stream)
 }
 
 static int launch_quant(const void *x, int dtype, int64_t n, const void *state, void *out, int mode,
-                        int sem, int use_state, hif8_stream_t stream, bool gelu = false)
+                        int sem, int use_state, hif8_stream_t stream, bool gelu = false, int parts = 0,
+                        float smax = 0.0f)
 {
     if (!x || !out || n <= 0 || (use_state && !state)) return HIF8_ERR_ARG;
     if (dtype != HIF8_DTYPE_BF16 && dtype != HIF8_DTYPE_F32 && !(dtype == kBF16F32 && mode != 2)) return HIF8_ERR_ARG;
@@ -1018,8 +1064,8 @@ static int launch_quant(const void *x, int dtype, int64_t n, const void *state, 
     if (!aligned16(x) || !aligned16(out)) return HIF8_ERR_ALIGN;
     const int wpc = mode == 0 ? kEncodeWgPerCu : kQdqWgPerCu;
     hipStream_t s = (hipStream_t)stream;
-    const State *st = (const State *)state;
-#define HIF8_LAUNCH(DT, MODE) launch_k_quant<DT, MODE>(x, n, st, out, sem, use_state, wpc, s)
+    State *st = (State *)state;   // written by a quantisation that settles it (parts > 0)
+#define HIF8_LAUNCH(DT, MODE) launch_k_quant<DT, MODE>(x, n, st, out, sem, use_state, wpc, s, parts, smax)
     if (gelu) {
         if (dtype != HIF8_DTYPE_BF16 || mode != 1 || !use_state) return HIF8_ERR_ARG;
         launch_gelu_quant(x, n, st, out, sem, s);
@@ -1039,6 +1085,29 @@ static int launch_quant(const void *x, int dtype, int64_t n, const void *state, 
     }
 #undef HIF8_LAUNCH
     return last_launch();
+}
+
+int hif8_quantize(const void *x, int dtype, int64_t n, float scale_max, void *state, void *out, int out_kind,
+                  int semantics, hif8_stream_t stream)
+{
+    if (!x || !state || !out || n <= 0) return HIF8_ERR_ARG;
+    if (dtype != HIF8_DTYPE_BF16 && dtype != HIF8_DTYPE_F32 && dtype != kBF16F32) return HIF8_ERR_ARG;
+    if (out_kind != HIF8_OUT_CODES && out_kind != HIF8_OUT_SAME && out_kind != HIF8_OUT_BF16) return HIF8_ERR_ARG;
+    if (semantics != HIF8_SEM_NPU && (semantics != HIF8_SEM_TORCH || out_kind == HIF8_OUT_CODES)) return HIF8_ERR_ARG;
+    if (!aligned16(x) || !aligned16(out)) return HIF8_ERR_ALIGN;
+    const int vec = dtype == HIF8_DTYPE_F32 ? 4 : 8;
+    const int cap = cu_count() * kAmaxWgPerCu;
+    const int grid = grid_for((n + vec * 8 - 1) / (vec * 8), cap < kMaxParts ? cap : kMaxParts);
+    hipStream_t s = (hipStream_t)stream;
+    if (dtype == HIF8_DTYPE_BF16)
+        hipLaunchKernelGGL((k_absmax<kBF16, true>), dim3(grid), dim3(kTPB), 0, s, x, n, (State *)state, scale_max);
+    else if (dtype == kBF16F32)
+        hipLaunchKernelGGL((k_absmax<kBF16F32, true>), dim3(grid), dim3(kTPB), 0, s, x, n, (State *)state, scale_max);
+    else
+        hipLaunchKernelGGL((k_absmax<kF32, true>), dim3(grid), dim3(kTPB), 0, s, x, n, (State *)state, scale_max);
+    const int rc = last_launch();
+    if (rc != HIF8_OK) return rc;
+    return launch_quant(x, dtype, n, state, out, out_kind, semantics, 1, stream, false, grid, scale_max);
 }
 
 int hif8_encode(const void *x, int dtype, int64_t n, const void *state, uint8_t *codes, hif8_stream_t stream)

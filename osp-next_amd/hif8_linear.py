@@ -44,13 +44,21 @@ class QuantState:
         self.device = torch.device(device)
         self.buf = _lib.new_state(self.device)
 
+    @classmethod
+    def unset(cls, device: torch.device) -> "QuantState":
+        """A state that only ``quantize`` may fill first (its buffer is not initialised)."""
+        st = object.__new__(cls)
+        st.device = device
+        st.buf = _lib.unset_state(device)
+        return st
+
     @property
     def ptr(self) -> int:
         return self.buf.data_ptr()
 
-    def scale(self) -> Tensor:
-        """The scale as a 0-dim fp32 device tensor (a copy; no host sync)."""
-        return self.buf[12:16].view(torch.float32).reshape(()).clone()
+    def scale(self, dtype: torch.dtype = torch.float32) -> Tensor:
+        """The scale as a 0-dim device tensor of ``dtype`` (a copy; no host sync)."""
+        return self.buf[12:16].view(torch.float32).reshape(()).to(dtype, copy=True)
 
     def read(self) -> Tuple[int, float]:
         """(amax bits, scale) on the host (synchronises the stream)."""
@@ -69,6 +77,13 @@ class QuantState:
 def _aligned(t: Tensor) -> Tensor:
     """The kernels use 128-bit accesses: realign offset views with one copy."""
     return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _bf16_bias(bias: Tensor) -> Tensor:
+    """The bias as the GEMMs take it: contiguous bf16 (the tensor itself where it is that already)."""
+    if bias.dtype == torch.bfloat16 and bias.is_contiguous():
+        return bias
+    return bias.detach().to(torch.bfloat16).contiguous()
 
 
 def _round_up(v: int, m: int) -> int:
@@ -179,12 +194,31 @@ def decode(codes: Tensor, state: QuantState, dtype: torch.dtype = torch.bfloat16
     return y
 
 
+def quantize(x: Tensor, scale_max: float, out_kind: int = _lib.OUT_SAME, semantics: int = _lib.SEM_NPU,
+             as_f32: bool = False) -> Tuple[Tensor, QuantState]:
+    """``absmax_scale`` into a fresh state, then ``encode`` (OUT_CODES), ``fake_quant`` (OUT_SAME) or
+    ``fake_quant_to_bf16`` (OUT_BF16) of a contiguous x, in two launches (hif8_quantize): the same bytes
+    and state."""
+    _lib.require_gpu_tensor(x, "x")
+    x = _aligned(x)
+    n = x.numel()
+    if n == 0:
+        raise ValueError("amax of an empty tensor")
+    dtype = _dtype_arg(x, as_f32)
+    if out_kind == _lib.OUT_SAME:
+        out = torch.empty_like(x)
+    else:
+        out = torch.empty(x.shape, dtype=torch.uint8 if out_kind == _lib.OUT_CODES else torch.bfloat16, device=x.device)
+    st = QuantState.unset(x.device)
+    _lib.check(_lib.load().hif8_quantize(x.data_ptr(), dtype, n, float(scale_max), st.ptr, out.data_ptr(), out_kind,
+                                         semantics, _lib.stream_ptr(x.device)), "hif8_quantize")
+    return out, st
+
+
 def _quant(x: Tensor, scale_max: float, semantics: int = _lib.SEM_NPU) -> Tuple[Tensor, Tensor]:
     """hif8_linear.py:42-50: returns ``(x_q, scale)``, scale a 0-dim tensor of x's dtype."""
-    xc = x.contiguous()
-    st = absmax_scale(xc, scale_max, QuantState(xc.device))
-    xq = fake_quant(xc, st, semantics)
-    return xq.view(x.shape), st.scale().to(x.dtype)
+    xq, st = quantize(x.contiguous(), scale_max, _lib.OUT_SAME, semantics)
+    return xq.view(x.shape), st.scale(x.dtype)
 
 
 # ------------------------------------------------------------ packed weight
@@ -201,8 +235,7 @@ class PackedWeight:
         w = weight.detach().contiguous()
         self.shape = tuple(w.shape)
         self.src_dtype = w.dtype
-        self.state = absmax_scale(w, scale_max, QuantState(w.device))
-        self.codes = encode(w, self.state)
+        self.codes, self.state = quantize(w, scale_max, _lib.OUT_CODES)
         self.scale_max = float(scale_max)
         self.key = (w.data_ptr(), weight._version, w.device)
         self._codes_t: Optional[Tensor] = None
@@ -407,7 +440,7 @@ def linear_fwd_wq_split(a: Tensor, w_q: Tensor, bias: Optional[Tensor] = None, s
     y = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
     b_ptr = None
     if bias is not None:
-        bias = bias.detach().to(torch.bfloat16).contiguous()
+        bias = _bf16_bias(bias)
         b_ptr = bias.data_ptr()
     need = L.hif8_linear_ksplit_workspace_bytes if wide else L.hif8_linear_split_workspace_bytes
     nbytes = int(need(M, N, K)) if split_tail else 0
@@ -452,7 +485,7 @@ def linear_fwd_wq(a: Tensor, w_q: Tensor, bias: Optional[Tensor], y_state: Optio
     y = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
     b_ptr = None
     if bias is not None:
-        bias = bias.detach().to(torch.bfloat16).contiguous()
+        bias = _bf16_bias(bias)
         b_ptr = bias.data_ptr()
     L = _lib.load()
     s = _lib.stream_ptr(a.device)
@@ -556,7 +589,7 @@ def linear_fwd(a: Tensor, a_fmt: int, a_state: Optional[QuantState], w: PackedWe
     y = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
     b_ptr = None
     if bias is not None:
-        bias = bias.detach().to(torch.bfloat16).contiguous()
+        bias = _bf16_bias(bias)
         b_ptr = bias.data_ptr()
     _lib.check(_lib.load().hif8_linear_fwd(a.data_ptr(), w.codes.data_ptr(), w.state.ptr, b_ptr, y.data_ptr(),
                                            M, N, K, _lib.stream_ptr(a.device)), "hif8_linear_fwd")
@@ -644,7 +677,7 @@ def linear_fwd_gelu_stat(a: Tensor, w: PackedWeight, bias: Optional[Tensor], y_s
     y = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
     b_ptr = None
     if bias is not None:
-        bias = bias.detach().to(torch.bfloat16).contiguous()
+        bias = _bf16_bias(bias)
         b_ptr = bias.data_ptr()
     _lib.check(_lib.load().hif8_linear_fwd_gelu_stat(a.data_ptr(), w.codes.data_ptr(), w.state.ptr, b_ptr,
                                                      y.data_ptr(), M, N, K, float(scale_max), y_state.ptr,
@@ -696,12 +729,9 @@ def quantize_activation(x2: Tensor, scale_max: float, a_format: str, as_f32: boo
     """Quantise a [M,K] activation for the fused GEMM: returns (a, a_fmt, state).  An fp32
     activation (or a bf16 one with ``as_f32``) is quantised in fp32 and handed over as its
     bf16 autocast rounding; ``a_format="codes"`` gives the 8-bit codes instead."""
-    st = absmax_scale(x2, scale_max, QuantState(x2.device), as_f32)
-    if a_format == "codes":
-        return encode(x2, st, as_f32), _lib.A_CODES, st
-    if x2.dtype == torch.bfloat16 and not as_f32:
-        return fake_quant(x2, st), _lib.A_BF16, st
-    return fake_quant_to_bf16(x2, st, as_f32=as_f32), _lib.A_BF16, st
+    kind = _lib.OUT_CODES if a_format == "codes" else _lib.OUT_BF16
+    a, st = quantize(x2, scale_max, kind, as_f32=as_f32)
+    return a, (_lib.A_CODES if a_format == "codes" else _lib.A_BF16), st
 
 
 # --------------------------------------------------------------- autograd
@@ -749,7 +779,7 @@ class _HIF8LinearFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         # x_q and w_q as the reference saves them (hif8_linear.py:78-82)
-        grad_q, _ = _quant(grad_output.contiguous(), ctx.smb)            # :93
+        grad_q, _ = quantize(grad_output.contiguous(), ctx.smb)           # :93
         g_2d = grad_q.reshape(-1, grad_q.shape[-1]).contiguous()
         M, N = g_2d.shape
         K = ctx.packed.shape[1]
@@ -809,11 +839,11 @@ class HIF8Linear(nn.Linear):
         self._prepacked = False
 
     def _packed_weight(self) -> PackedWeight:
-        w = self.weight
-        key = (w.data_ptr(), w._version, w.device)
         p = self._packed
         if self._prepacked and p is not None:
             return p
+        w = self.weight
+        key = (w.data_ptr(), w._version, w.device)
         if p is None or p.key != key or p.scale_max != float(self.scale_max_forward):
             p = PackedWeight(w, self.scale_max_forward)
             self._packed = p
