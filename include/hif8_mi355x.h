@@ -103,6 +103,11 @@ int hif8_set_scale(void *state, int dtype, float scale, hif8_stream_t stream);
 #define HIF8_OUT_BF16 3
 int hif8_quantize(const void *x, int dtype, int64_t n, float scale_max, void *state, void *out, int out_kind,
                   int semantics, hif8_stream_t stream);
+/* hif8_quantize with HIF8_OUT_BF16 (NPU semantics) and the codes from the same pass: what a training step
+ * keeps of an fp32 input (its codes, for the backward's fp32 x_q) beside the GEMM operand.  dtype
+ * HIF8_DTYPE_F32 or HIF8_DTYPE_BF16_AS_F32; codes 16-byte aligned. */
+int hif8_quantize_with_codes(const void *x, int dtype, int64_t n, float scale_max, void *state, uint16_t *x_q,
+                             uint8_t *codes, hif8_stream_t stream);
 
 /* ---------------------------------------------------------------------------
  * Encode: HiF8 codes of qdq(x * scale), NPU semantics (hif8_linear.py:47-48 with
@@ -334,7 +339,8 @@ int64_t hif8_linear_ksplit_workspace_bytes(int64_t M, int64_t N, int64_t K);
  *   hif8_linear_wgrad_scaled: dw[n_out, k_in] = g[tokens, n_out]^T . v[tokens, k_in] / scale
  *   hif8_linear_fwd_scaled:   y[M, N] = a[M, K] . v[N, K]^T / scale
  * with fp32 sums of exact products and the scale of the state of the tensor v was encoded from, one
- * division per output; out_dtype HIF8_DTYPE_F32 or HIF8_DTYPE_BF16 (RNE).  Shapes and alignment as
+ * division per output; v_state NULL in hif8_linear_fwd_scaled: scale 1, a . v^T itself (the fp32
+ * gradient of an fp32 input, from a bf16 w_q).  out_dtype HIF8_DTYPE_F32 or HIF8_DTYPE_BF16 (RNE).  Shapes and alignment as
  * hif8_linear_wgrad (tokens below 2^22) and hif8_linear_fwd_wq; workspace NULL, or
  * hif8_linear_ksplit_workspace_bytes (n_out, k_in, tokens or M, N, K) bytes. */
 int hif8_linear_wgrad_scaled(const uint16_t *g, const uint16_t *v, const void *v_state, void *dw, int out_dtype,

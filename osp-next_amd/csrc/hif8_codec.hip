@@ -153,7 +153,7 @@ __global__ __launch_bounds__(kTPB) void k_absmax(const void *__restrict__ xv, in
 
 // Element j of k_quant through the scalar reference route.
 template <int DT, int MODE>
-__device__ __forceinline__ void scalar_elem(const void *xv, void *outv, int64_t j, float s, int sem)
+__device__ __forceinline__ void scalar_elem(const void *xv, void *outv, uint8_t *codes_out, int64_t j, float s, int sem)
 {
     uint32_t xb, yb, code;
     if (DT == kBF16) {
@@ -164,6 +164,7 @@ __device__ __forceinline__ void scalar_elem(const void *xv, void *outv, int64_t 
         slow_elem<kF32>(xb, s, sem, yb, code);
         if (MODE == 3) yb = f2bf(u2f(yb));
     }
+    if (MODE == 3 && codes_out) codes_out[j] = uint8_t(code);
     if (MODE == 0) ((uint8_t *)outv)[j] = uint8_t(code);
     else if (DT == kBF16 || MODE == 3) ((uint16_t *)outv)[j] = uint16_t(yb);
     else ((uint32_t *)outv)[j] = yb;
@@ -178,10 +179,12 @@ __device__ __forceinline__ void scalar_elem(const void *xv, void *outv, int64_t 
 // parts > 0: the amax, scale and decode tables come from the parts workgroup maxima that k_absmax<DT, true>
 // left in st, reduced by every workgroup for itself; workgroup 0 writes them into st as an amax pass
 // settles it, counters included (st may have been uninitialised).
+// codes_out (MODE 3): the codes as MODE 0 writes them, from the same pass.
 template <int DT, int MODE, int TPB = kTPB>
 __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int64_t n,
                                                  State *st, void *__restrict__ outv,
-                                                 int sem, int use_state, int span, int parts, float smax)
+                                                 int sem, int use_state, int span, int parts, float smax,
+                                                 uint8_t *__restrict__ codes_out)
 {
     __shared__ __attribute__((aligned(16))) uint8_t lds[kLdsBytes];
     const int tid = threadIdx.x;
@@ -366,16 +369,17 @@ __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int6
                         if (wide[t] > 0x7F80u) codes[t >> 2] = (codes[t >> 2] & ~(0xFFu << (8 * (t & 3)))) | (kNanCode << (8 * (t & 3)));
                 }
             }
-            if (MODE == 0) {
+            if (MODE == 0 || (MODE == 3 && codes_out)) {
                 // chunk j's kIpc codes are bytes j * kIpc .. of codes[]
+                void *co = MODE == 0 ? outv : codes_out;
 #pragma unroll
                 for (int j = 0; j < kVec; ++j) {
                     const int64_t c = G0 * kVec + j * TPB + tid;
                     if (c >= nchunk) continue;
-                    if (kIpc == 8) st_stream(&((u32x2 *)outv)[c], u32x2{codes[2 * j], codes[2 * j + 1]});
-                    else st_stream(&((uint32_t *)outv)[c], codes[j]);
+                    if (kIpc == 8) st_stream(&((u32x2 *)co)[c], u32x2{codes[2 * j], codes[2 * j + 1]});
+                    else st_stream(&((uint32_t *)co)[c], codes[j]);
                 }
-                continue;
+                if (MODE == 0) continue;
             }
             // qdq output through the decode table
             uint32_t y[16];
@@ -426,11 +430,11 @@ __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int6
         // degenerate scale (amax Inf/NaN, scale 0/Inf/NaN): element-wise reference route, a
         // grid-stride loop over the elements (each visited once whatever the grid)
         for (int64_t j = int64_t(blockIdx.x) * TPB + tid; j < (ngrp << 4); j += stride)
-            scalar_elem<DT, MODE>(xv, outv, j, s, sem);
+            scalar_elem<DT, MODE>(xv, outv, codes_out, j, s, sem);
     }
     // tail (n % 16) through the scalar route
     for (int64_t j = (ngrp << 4) + int64_t(blockIdx.x) * TPB + tid; j < n; j += stride)
-        scalar_elem<DT, MODE>(xv, outv, j, s, sem);
+        scalar_elem<DT, MODE>(xv, outv, codes_out, j, s, sem);
 }
 
 // QFuncs/hif8.py:6-23 evaluated on a bf16 tensor without force_fp32 (quant_dequant_float with
@@ -948,7 +952,7 @@ template <int DT, int MODE> static int resident_wgs()
 
 template <int DT, int MODE>
 static void launch_k_quant(const void *x, int64_t n, State *st, void *out, int sem, int use_state, int wg_per_cu,
-                           hipStream_t s, int parts = 0, float smax = 0.0f)
+                           hipStream_t s, int parts = 0, float smax = 0.0f, uint8_t *codes = nullptr)
 {
     const int64_t ngrp = (n + 15) / 16;
     int grid, span = 0;
@@ -962,7 +966,7 @@ static void launch_k_quant(const void *x, int64_t n, State *st, void *out, int s
         grid = grid_for(ngrp, cu_count() * (wg_per_cu < fit ? wg_per_cu : fit));
     }
     hipLaunchKernelGGL((k_quant<DT, MODE>), dim3(grid), dim3(kTPB), 0, s, x, n, st, out, sem, use_state, span,
-                       parts, smax);
+                       parts, smax, codes);
 }
 
 // The GELU route: the prep kernel, then spans of HIF8_GELU_SPAN x 256 groups per workgroup
@@ -1056,7 +1060,7 @@ int hif8_set_scale(void *state, int dtype, float scale, hif8_stream_t stream)
 
 static int launch_quant(const void *x, int dtype, int64_t n, const void *state, void *out, int mode,
                         int sem, int use_state, hif8_stream_t stream, bool gelu = false, int parts = 0,
-                        float smax = 0.0f)
+                        float smax = 0.0f, uint8_t *codes = nullptr)
 {
     if (!x || !out || n <= 0 || (use_state && !state)) return HIF8_ERR_ARG;
     if (dtype != HIF8_DTYPE_BF16 && dtype != HIF8_DTYPE_F32 && !(dtype == kBF16F32 && mode != 2)) return HIF8_ERR_ARG;
@@ -1065,7 +1069,7 @@ static int launch_quant(const void *x, int dtype, int64_t n, const void *state, 
     const int wpc = mode == 0 ? kEncodeWgPerCu : kQdqWgPerCu;
     hipStream_t s = (hipStream_t)stream;
     State *st = (State *)state;   // written by a quantisation that settles it (parts > 0)
-#define HIF8_LAUNCH(DT, MODE) launch_k_quant<DT, MODE>(x, n, st, out, sem, use_state, wpc, s, parts, smax)
+#define HIF8_LAUNCH(DT, MODE) launch_k_quant<DT, MODE>(x, n, st, out, sem, use_state, wpc, s, parts, smax, codes)
     if (gelu) {
         if (dtype != HIF8_DTYPE_BF16 || mode != 1 || !use_state) return HIF8_ERR_ARG;
         launch_gelu_quant(x, n, st, out, sem, s);
@@ -1087,14 +1091,14 @@ static int launch_quant(const void *x, int dtype, int64_t n, const void *state, 
     return last_launch();
 }
 
-int hif8_quantize(const void *x, int dtype, int64_t n, float scale_max, void *state, void *out, int out_kind,
-                  int semantics, hif8_stream_t stream)
+static int quantize(const void *x, int dtype, int64_t n, float scale_max, void *state, void *out, int out_kind,
+                    int semantics, uint8_t *codes, hif8_stream_t stream)
 {
     if (!x || !state || !out || n <= 0) return HIF8_ERR_ARG;
     if (dtype != HIF8_DTYPE_BF16 && dtype != HIF8_DTYPE_F32 && dtype != kBF16F32) return HIF8_ERR_ARG;
     if (out_kind != HIF8_OUT_CODES && out_kind != HIF8_OUT_SAME && out_kind != HIF8_OUT_BF16) return HIF8_ERR_ARG;
     if (semantics != HIF8_SEM_NPU && (semantics != HIF8_SEM_TORCH || out_kind == HIF8_OUT_CODES)) return HIF8_ERR_ARG;
-    if (!aligned16(x) || !aligned16(out)) return HIF8_ERR_ALIGN;
+    if (!aligned16(x) || !aligned16(out) || !aligned16(codes)) return HIF8_ERR_ALIGN;
     const int vec = dtype == HIF8_DTYPE_F32 ? 4 : 8;
     const int cap = cu_count() * kAmaxWgPerCu;
     const int grid = grid_for((n + vec * 8 - 1) / (vec * 8), cap < kMaxParts ? cap : kMaxParts);
@@ -1107,7 +1111,20 @@ int hif8_quantize(const void *x, int dtype, int64_t n, float scale_max, void *st
         hipLaunchKernelGGL((k_absmax<kF32, true>), dim3(grid), dim3(kTPB), 0, s, x, n, (State *)state, scale_max);
     const int rc = last_launch();
     if (rc != HIF8_OK) return rc;
-    return launch_quant(x, dtype, n, state, out, out_kind, semantics, 1, stream, false, grid, scale_max);
+    return launch_quant(x, dtype, n, state, out, out_kind, semantics, 1, stream, false, grid, scale_max, codes);
+}
+
+int hif8_quantize(const void *x, int dtype, int64_t n, float scale_max, void *state, void *out, int out_kind,
+                  int semantics, hif8_stream_t stream)
+{
+    return quantize(x, dtype, n, scale_max, state, out, out_kind, semantics, nullptr, stream);
+}
+
+int hif8_quantize_with_codes(const void *x, int dtype, int64_t n, float scale_max, void *state, uint16_t *x_q,
+                             uint8_t *codes, hif8_stream_t stream)
+{
+    if (!codes || (dtype != HIF8_DTYPE_F32 && dtype != kBF16F32)) return HIF8_ERR_ARG;
+    return quantize(x, dtype, n, scale_max, state, x_q, HIF8_OUT_BF16, HIF8_SEM_NPU, codes, stream);
 }
 
 int hif8_encode(const void *x, int dtype, int64_t n, const void *state, uint8_t *codes, hif8_stream_t stream)

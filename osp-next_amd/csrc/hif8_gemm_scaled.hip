@@ -33,7 +33,7 @@ __global__ __launch_bounds__(kThreads) void k_split_reduce_scaled(const float *_
     tile_origin(full_tiles + int(tile), tiles_m, tiles_n, group_m, m0, n0);
     const uint32_t wm = (wave & 1u) * 128u, wn = (wave >> 1) * 128u;
     const f32x4 *P = (const f32x4 *)part + size_t(tile) * size_t(splits) * 16384u + wave * 4096u + lane;
-    const Divisor d(st->scale);
+    const Divisor d(st ? st->scale : 1.0f);
     const int n = n0 + int(wn) + i * 16 + int(4u * g);
     if (n >= N) return;
     for (int j = 0; j < 8; ++j) {
@@ -121,7 +121,7 @@ extern "C" int hif8_linear_fwd_scaled(const uint16_t *a, const uint16_t *w, cons
                                       int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes,
                                       hif8_stream_t stream)
 {
-    if (!a || !w || !w_state || !y) return HIF8_ERR_ARG;
+    if (!a || !w || !y) return HIF8_ERR_ARG;
     if (M <= 0 || N <= 0 || K <= 0) return HIF8_ERR_ARG;
     if (out_dtype != HIF8_DTYPE_BF16 && out_dtype != HIF8_DTYPE_F32) return HIF8_ERR_ARG;
     if (M >= (int64_t(1) << 31) || N >= (int64_t(1) << 31) || K >= (int64_t(1) << 22)) return HIF8_ERR_SHAPE;

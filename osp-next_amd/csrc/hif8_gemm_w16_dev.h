@@ -240,7 +240,7 @@ __device__ __forceinline__ void tile_origin(int t, int tiles_m, int tiles_n, int
 // lane order) for k_split_reduce.  (A separate instantiation: in the same kernel as the bf16
 // epilogue, the register allocator moved all accumulators to VGPRs ahead of the branch and
 // spilled.)
-// EPI 3: y = acc / scale, no bias, with the scale of the state y_st: one of the operands holds the
+// EPI 3: y = acc / scale, no bias, with the scale of the state y_st (1 without one): one of the operands holds the
 // raw HiF8 values of codes instead of their quotients by the scale.  y is fp32 when splits != 0, else
 // bf16.
 // TR: X and Wq are k-major, X^T [K][M] and Wq^T [K][N] (contiguous rows of M and N elements):
@@ -437,7 +437,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_linear_w16(const uint16_t *__re
     }
     if (EPI == 3) {
         // straight from the accumulators: 4 consecutive features per lane, 16 (fp32) or 8 bytes
-        const Divisor d(y_st->scale);
+        const Divisor d(y_st ? y_st->scale : 1.0f);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int n = n0 + int(wn) + i * 16 + int(4u * g);

@@ -215,6 +215,21 @@ def quantize(x: Tensor, scale_max: float, out_kind: int = _lib.OUT_SAME, semanti
     return out, st
 
 
+def quantize_with_codes(x: Tensor, scale_max: float) -> Tuple[Tensor, Tensor, QuantState]:
+    """(bf16 x_q, codes, state) of a contiguous fp32 x in two launches (hif8_quantize_with_codes)."""
+    _lib.require_gpu_tensor(x, "x")
+    x = _aligned(x)
+    if x.numel() == 0:
+        raise ValueError("amax of an empty tensor")
+    xq = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
+    codes = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
+    st = QuantState.unset(x.device)
+    _lib.check(_lib.load().hif8_quantize_with_codes(x.data_ptr(), _lib.dtype_code(x.dtype), x.numel(),
+                                                    float(scale_max), st.ptr, xq.data_ptr(), codes.data_ptr(),
+                                                    _lib.stream_ptr(x.device)), "hif8_quantize_with_codes")
+    return xq, codes, st
+
+
 def _quant(x: Tensor, scale_max: float, semantics: int = _lib.SEM_NPU) -> Tuple[Tensor, Tensor]:
     """hif8_linear.py:42-50: returns ``(x_q, scale)``, scale a 0-dim tensor of x's dtype."""
     xq, st = quantize(x.contiguous(), scale_max, _lib.OUT_SAME, semantics)
@@ -289,8 +304,9 @@ def dgrad_fused_ok(grad_q: Tensor, w: "PackedWeight") -> bool:
     return grad_q.dtype == torch.bfloat16 and w.src_dtype == torch.bfloat16 and _round_up(N, 64) < (1 << 22)
 
 
-def linear_dgrad(grad_q2: Tensor, w: "PackedWeight") -> Tensor:
-    """grad_q [M, N] @ w_q [N, K] -> [M, K] bf16 (hif8_linear.py:97): the forward GEMM with the
+def linear_dgrad(grad_q2: Tensor, w: "PackedWeight", out_dtype: torch.dtype = torch.bfloat16) -> Tensor:
+    """grad_q [M, N] @ w_q [N, K] -> [M, K] bf16 (hif8_linear.py:97; ``out_dtype`` fp32 for the
+    gradient of an fp32 input, on the decode-once route without the rounding to bf16): the forward GEMM with the
     transposed weight codes [K, N] as its weight, on the route the forward takes at this M (the
     fused GEMM, or the transposed codes decoded once and the decode-free GEMM with its last
     partial wave of tiles split over k ranges).  The reduction (N) is padded to a multiple of 64
@@ -303,12 +319,20 @@ def linear_dgrad(grad_q2: Tensor, w: "PackedWeight") -> Tensor:
         g = pad_2d(g, M, Np)
     codes_t = w.codes_t() if (Np, Kp) == (N, K) else w.codes_t_padded(Kp, Np)
     if decode_once(M, Np):
-        y = linear_fwd_wq_split(g, decode(codes_t, w.state, torch.bfloat16))
+        w_qt = decode(codes_t, w.state, torch.bfloat16)
+        if out_dtype == torch.float32:
+            y = torch.empty((M, Kp), dtype=torch.float32, device=g.device)
+            _lib.check(_lib.load().hif8_linear_fwd_scaled(g.data_ptr(), w_qt.data_ptr(), None, y.data_ptr(),
+                                                          _lib.DTYPE_F32, M, Kp, Np, None, 0,
+                                                          _lib.stream_ptr(g.device)), "hif8_linear_fwd_scaled")
+        else:
+            y = linear_fwd_wq_split(g, w_qt)
     else:
         y = torch.empty((M, Kp), dtype=torch.bfloat16, device=g.device)
         _lib.check(_lib.load().hif8_linear_fwd(g.data_ptr(), codes_t.data_ptr(), w.state.ptr, None, y.data_ptr(),
                                                M, Kp, Np, _lib.stream_ptr(g.device)), "hif8_linear_fwd (dgrad)")
-    return y if Kp == K else pad_2d(y, M, K)
+    y = y if Kp == K else pad_2d(y, M, K)
+    return y.to(out_dtype)
 
 
 def transpose_bf16(x2: Tensor, rows_pad: Optional[int] = None) -> Tensor:
@@ -762,12 +786,15 @@ class _HIF8LinearFunction(torch.autograd.Function):
         if packed is None:
             packed = PackedWeight(weight, scale_max_forward)
         needs_grad = any(ctx.needs_input_grad[:3])
-        a, a_fmt, a_st = quantize_activation(x2, scale_max_forward, "codes" if a_format == "codes" else "bf16")
-        y = linear_any(a, a_fmt, a_st, packed, bias)
+        if needs_grad and x.dtype != torch.bfloat16 and a_format != "codes":
+            # the backward's x_q is the fp32 one (hif8_linear.py:78-82): keep its codes
+            x_q, a, a_st = quantize_with_codes(x2, scale_max_forward)
+            a_fmt = _lib.A_CODES
+            y = linear_any(x_q, _lib.A_BF16, None, packed, bias)
+        else:
+            a, a_fmt, a_st = quantize_activation(x2, scale_max_forward, "codes" if a_format == "codes" else "bf16")
+            y = linear_any(a, a_fmt, a_st, packed, bias)
         if needs_grad:
-            if x.dtype != torch.bfloat16 and a_fmt == _lib.A_BF16:
-                # the backward's x_q is the fp32 one (hif8_linear.py:78-82): keep its codes
-                a, a_fmt = encode(x2, a_st), _lib.A_CODES
             ctx.a, ctx.a_fmt, ctx.a_st, ctx.packed = a, a_fmt, a_st, packed
             ctx.x_dtype, ctx.w_dtype = x.dtype, weight.dtype
             ctx.x_shape = x.shape
@@ -785,7 +812,7 @@ class _HIF8LinearFunction(torch.autograd.Function):
         K = ctx.packed.shape[1]
         g_bf16 = g_2d.dtype == torch.bfloat16
         if dgrad_fused_ok(g_2d, ctx.packed):                              # :97, grad_q @ w_q
-            grad_input = linear_dgrad(g_2d, ctx.packed)
+            grad_input = linear_dgrad(g_2d, ctx.packed, ctx.x_dtype)
         else:                                                             # w_q fp32
             grad_input = None
             if g_bf16 and ctx.packed.src_dtype == ctx.w_dtype == torch.float32:

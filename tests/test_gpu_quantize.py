@@ -73,6 +73,18 @@ def test_bf16_as_f32(pkg, n):
         both(pkg, inputs(n, torch.bfloat16, None, 3), kind, 0, as_f32=True)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 17, 4099, SPAN + 333])
+@pytest.mark.parametrize("special", [None, "inf", "nan", "zeros"])
+def test_with_codes(pkg, n, special):
+    """The bf16 x_q and the codes of one pass: those of the two separate passes."""
+    x = inputs(n, torch.float32, special, n)
+    xq, codes, st = pkg.hif8_linear.quantize_with_codes(x, 15.0)
+    want = pkg.absmax_scale(x, 15.0, pkg.QuantState(DEV))
+    assert torch.equal(codes, pkg.encode(x, want)) and st.read()[0] == want.read()[0]
+    assert torch.equal(xq.view(torch.int16), pkg.fake_quant_to_bf16(x, want).view(torch.int16))
+
+
 def test_status_codes_without_gpu(pkg):
     L = pkg._lib.load()
     f = 0x100000
@@ -80,4 +92,7 @@ def test_status_codes_without_gpu(pkg):
     def q(x=f, dt=0, n=16, st=f, out=f, kind=1, sem=0):
         return L.hif8_quantize(x, dt, n, 15.0, st, out, kind, sem, None)
     assert q(x=None) == -1 and q(st=None) == -1 and q(out=None) == -1 and q(n=0) == -1 and q(dt=7) == -1
+    assert L.hif8_quantize_with_codes(f, 1, 16, 15.0, f, f, None, None) == -1
+    assert L.hif8_quantize_with_codes(f, 0, 16, 15.0, f, f, f, None) == -1        # a bf16 tensor's x_q is bf16
+    assert L.hif8_quantize_with_codes(f, 1, 16, 15.0, f, f, f + 4, None) == -3
     assert q(kind=2) == -1 and q(sem=2) == -1 and q(kind=0, sem=1) == -1 and q(x=f + 2) == -3 and q(out=f + 8) == -3

@@ -73,6 +73,18 @@ def test_dgrad_scaled(pkg, M, N, K, out_dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(8192, 2112, 40), (8200, 2304, 264), (24600, 64, 8), (8193, 2100, 36)])
+def test_dgrad_fp32_output(pkg, M, N, K):
+    """The gradient of an fp32 input with a bf16 weight on the decode-once route: fp32, unrounded."""
+    print(f"[scaled] dgrad fp32 M={M} N={N} K={K}", flush=True)
+    assert pkg.hif8_linear.decode_once(M, -(-N // 64) * 64)
+    g = torch.Generator().manual_seed(M + N + K)
+    gq, _ = pkg._quant(torch.randn(M, N, generator=g).to(torch.bfloat16).to(DEV), 224.0)
+    packed = pkg.PackedWeight((torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16).to(DEV), 15.0)
+    bound(pkg.linear_dgrad(gq, packed, torch.float32), gq, packed.dequantize(torch.bfloat16), torch.float32)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 def test_wgrad_scaled_non_finite_input(pkg, value):
     """An Inf or NaN in x makes the scale 0 or NaN and every quotient non-finite: outputs are NaN or
@@ -138,6 +150,6 @@ def test_scaled_status_codes_without_gpu(pkg):
         return L.hif8_linear_fwd_scaled(a, fake, st, y, dt, M, N, K, None, 0, None)
     assert wg(g=None) == -1 and wg(st=None) == -1 and wg(dt=2) == -1 and wg(tokens=0) == -1
     assert wg(n=260) == -2 and wg(k=100) == -2 and wg(tokens=1 << 22) == -2 and wg(dw=fake + 2) == -3
-    assert fw(a=None) == -1 and fw(st=None) == -1 and fw(dt=3) == -1 and fw(N=0) == -1
+    assert fw(a=None) == -1 and fw(dt=3) == -1 and fw(N=0) == -1
     assert fw(K=100) == -2 and fw(N=100) == -2 and fw(K=1 << 22) == -2 and fw(y=fake + 8) == -3
     assert L.hif8_decode_values(None, 16, fake, None) == -1 and L.hif8_decode_values(fake, 16, fake + 4, None) == -3
