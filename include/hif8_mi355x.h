@@ -108,6 +108,15 @@ int hif8_quantize(const void *x, int dtype, int64_t n, float scale_max, void *st
  * HIF8_DTYPE_F32 or HIF8_DTYPE_BF16_AS_F32; codes 16-byte aligned. */
 int hif8_quantize_with_codes(const void *x, int dtype, int64_t n, float scale_max, void *state, uint16_t *x_q,
                              uint8_t *codes, hif8_stream_t stream);
+/* hif8_quantize of a bf16 gradient [rows, cols] (HIF8_OUT_SAME, NPU semantics) with the sums of x_q's
+ * columns, the bias gradient grad_q.sum(0) of hif8_linear.py:107: fp32 sums in a fixed order, written as
+ * fp32 or bf16 (RNE).  cols % 8 == 0; x, x_q and the workspace (hif8_quantize_colsum_workspace_bytes
+ * (rows, cols)) 16-byte aligned. */
+int64_t hif8_quantize_colsum_workspace_bytes(int64_t rows, int64_t cols);
+int hif8_quantize_colsum(const uint16_t *x, int64_t rows, int64_t cols, float scale_max, void *state, uint16_t *x_q,
+                         void *colsum, int colsum_dtype, void *workspace, int64_t workspace_bytes,
+                         hif8_stream_t stream);
+
 
 /* ---------------------------------------------------------------------------
  * Encode: HiF8 codes of qdq(x * scale), NPU semantics (hif8_linear.py:47-48 with

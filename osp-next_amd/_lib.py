@@ -33,6 +33,8 @@ SIGNATURES = {
     "hif8_set_scale": (_i, [_p, _i, _f, _p]),
     "hif8_quantize": (_i, [_p, _i, _i64, _f, _p, _p, _i, _i, _p]),
     "hif8_quantize_with_codes": (_i, [_p, _i, _i64, _f, _p, _p, _p, _p]),
+    "hif8_quantize_colsum_workspace_bytes": (_i64, [_i64, _i64]),
+    "hif8_quantize_colsum": (_i, [_p, _i64, _i64, _f, _p, _p, _p, _i, _p, _i64, _p]),
     "hif8_encode": (_i, [_p, _i, _i64, _p, _p, _p]),
     "hif8_fake_quant": (_i, [_p, _i, _i64, _p, _p, _i, _p]),
     "hif8_fake_quant_to_bf16": (_i, [_p, _i, _i64, _p, _p, _i, _p]),

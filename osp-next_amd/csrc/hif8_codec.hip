@@ -151,6 +151,35 @@ __global__ __launch_bounds__(kTPB) void k_absmax(const void *__restrict__ xv, in
     else fold_amax(st, m, gridDim.x, DT, smax, red + kTPB / 64);
 }
 
+// The scale of a tensor whose amax pass left `parts` workgroup maxima in st (256 threads, `red` 4 words of
+// LDS); with `settle` (one workgroup of the grid) also written into st with its tables, flags and zero
+// counters, as an amax pass settles it.
+__device__ __forceinline__ float parts_scale(State *st, int parts, int dt, float smax, bool settle, uint32_t *red,
+                                             bool &fast)
+{
+    const int tid = threadIdx.x;
+    uint32_t m = tid < parts ? amax_parts(st)[tid] : 0u;
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
+    if ((tid & 63) == 0) red[tid >> 6] = m;
+    __syncthreads();
+    m = max(max(red[0], red[1]), max(red[2], red[3]));
+    const float s = scale_from_amax(m, dt, smax, fast);
+    if (settle) {
+        init_state(st);
+        __syncthreads();
+        if (tid == 0) write_amax_state(st, m, dt, smax);
+        fill_luts(st, s, uint32_t(tid));
+    }
+    return s;
+}
+// fill_luts into a quantise kernel's LDS (256 threads)
+__device__ __forceinline__ void parts_luts(uint8_t *lds, float s)
+{
+    const float y = u2f(decode_bits(threadIdx.x)) / s;
+    ((float *)(lds + kLdsLutF32))[threadIdx.x] = y;
+    ((uint16_t *)(lds + kLdsLutBf16))[threadIdx.x] = uint16_t(f2bf(y));
+}
+
 // Element j of k_quant through the scalar reference route.
 template <int DT, int MODE>
 __device__ __forceinline__ void scalar_elem(const void *xv, void *outv, uint8_t *codes_out, int64_t j, float s, int sem)
@@ -216,22 +245,9 @@ __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int6
     float s;
     bool fast, nan_guard;
     if (MODE != 2 && parts > 0) {
-        uint32_t m = tid < parts ? amax_parts(st)[tid] : 0u;
-        for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 64));
         __shared__ uint32_t red[TPB / 64];
-        if ((tid & 63) == 0) red[tid >> 6] = m;
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < TPB / 64; ++w) m = max(m, red[w]);
-        constexpr int kStateDt = DT == kBF16 ? kBF16 : kF32;
-        s = scale_from_amax(m, kStateDt, smax, fast);
+        s = parts_scale(st, parts, DT == kBF16 ? kBF16 : kF32, smax, blockIdx.x == 0, red, fast);
         nan_guard = !fast;
-        if (blockIdx.x == 0) {
-            init_state(st);
-            __syncthreads();
-            if (tid == 0) write_amax_state(st, m, kStateDt, smax);
-            if (tid < 256) fill_luts(st, s, uint32_t(tid));
-        }
     } else {
         s = use_state ? st->scale : 1.0f;
         fast = use_state ? (st->fast != 0) : true;
@@ -241,11 +257,7 @@ __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int6
     }
     // decode tables for this scale
     if (MODE != 2 && parts > 0) {
-        if (tid < 256) {
-            const float y = u2f(decode_bits(uint32_t(tid))) / s;
-            ((float *)(lds + kLdsLutF32))[tid] = y;
-            ((uint16_t *)(lds + kLdsLutBf16))[tid] = uint16_t(f2bf(y));
-        }
+        parts_luts(lds, s);
     } else if (tid < 256) {
         uint32_t c = uint32_t(tid);
         float y;
@@ -435,6 +447,105 @@ __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int6
     // tail (n % 16) through the scalar route
     for (int64_t j = (ngrp << 4) + int64_t(blockIdx.x) * TPB + tid; j < n; j += stride)
         scalar_elem<DT, MODE>(xv, outv, codes_out, j, s, sem);
+}
+
+// The fake quant of a bf16 gradient [rows, cols] (NPU semantics) with the column sums of its result, which
+// are the bias gradient (hif8_linear.py:93,107): a sum over g_q as a pass of its own reads it all again
+// (106 us for [32760, 8960], the copy rate).  A workgroup takes `width` 16-byte chunks of the columns
+// (blockIdx.x) by rpw rows (blockIdx.y): a thread keeps one chunk's 8 columns, its sums in registers,
+// kColRows rows in flight, and leaves them in part[blockIdx.y][cols] for k_colsum_reduce.  The scale
+// comes from the amax pass's parts as in k_quant.  With amax and reduction (us), against hif8_quantize and
+// torch's sum: [32760, 8960] 326 against 280 + 111, [32760, 1536] 65 against 53 + 39, [75600, 5120] 458 against 366 + 149,
+// [500, 1536] 16 against 11 + 15.  It is bound by its arithmetic and table lookups (5.0 TB/s against the plain pass's 6.1).
+constexpr int kColRows = 8;
+__global__ __launch_bounds__(kTPB) void k_quant_cols(const uint16_t *__restrict__ x, int64_t rows, int64_t cols,
+                                                      State *st, uint16_t *__restrict__ xq, int parts, float smax,
+                                                      int width, int rpw, float *__restrict__ part)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kLdsBytes];
+    __shared__ uint32_t red[kTPB / 64];
+    const int tid = threadIdx.x;
+    const int64_t cpr = cols >> 3, c = int64_t(blockIdx.x) * width + tid;
+    const bool live = tid < width && c < cpr;
+    const int64_t r0 = int64_t(blockIdx.y) * rpw, r1 = r0 + rpw < rows ? r0 + rpw : rows;
+    const u32x4 *src = (const u32x4 *)x + c;
+    u32x4 *dst = (u32x4 *)xq + c;
+    bool fast;
+    const float s = parts_scale(st, parts, kBF16, smax, blockIdx.x == 0 && blockIdx.y == 0, red, fast);
+    parts_luts(lds, s);
+    {
+        const uint4 *et = (const uint4 *)&kEncTable;
+        uint4 *d = (uint4 *)(lds + kTabLo);
+        for (uint32_t i = tid; i < sizeof(EncTable) / 16; i += kTPB) d[i] = et[i];
+    }
+    __syncthreads();
+    if (!live) return;
+    const uint16_t *lut16 = (const uint16_t *)(lds + kLdsLutBf16);
+    float sum[8] = {};
+    for (int64_t r = r0; r < r1; r += kColRows) {
+        u32x4 v[kColRows];
+#pragma unroll
+        for (int k = 0; k < kColRows; ++k)
+            v[k] = r + k < r1 ? ld_stream(src + (r + k) * cpr) : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int k = 0; k < kColRows; ++k) {
+            u32x4 o;
+            if (fast) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t p0 = v[k][2 * h], p1 = v[k][2 * h + 1];
+                    const uint32_t q01 = f2bf_pk(u2f(p0 << 16) * s, u2f(p0 & 0xFFFF0000u) * s);
+                    const uint32_t q23 = f2bf_pk(u2f(p1 << 16) * s, u2f(p1 & 0xFFFF0000u) * s);
+                    const uint32_t mags = uint32_t(lds[clampu(q01 & 0x7FFFu)]) | (uint32_t(lds[clampu((q01 >> 16) & 0x7FFFu)]) << 8) |
+                                          (uint32_t(lds[clampu(q23 & 0x7FFFu)]) << 16) | (uint32_t(lds[clampu((q23 >> 16) & 0x7FFFu)]) << 24);
+                    const uint32_t d = apply_signs(mags, __builtin_amdgcn_perm(p1, p0, 0x07050301u) & 0x80808080u);
+                    o[2 * h] = uint32_t(lut16[d & 0xFFu]) | (uint32_t(lut16[(d >> 8) & 0xFFu]) << 16);
+                    o[2 * h + 1] = uint32_t(lut16[(d >> 16) & 0xFFu]) | (uint32_t(lut16[d >> 24]) << 16);
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    uint32_t y0, y1, code;
+                    slow_elem<kBF16>(v[k][t] & 0xFFFFu, s, kSemNpu, y0, code);
+                    slow_elem<kBF16>(v[k][t] >> 16, s, kSemNpu, y1, code);
+                    o[t] = y0 | (y1 << 16);
+                }
+            }
+            if (r + k >= r1) continue;
+            st_stream(dst + (r + k) * cpr, o);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                sum[2 * t] += u2f(o[t] << 16);
+                sum[2 * t + 1] += u2f(o[t] & 0xFFFF0000u);
+            }
+        }
+    }
+    float *p = part + int64_t(blockIdx.y) * cols + 8 * c;
+    *(float4 *)p = make_float4(sum[0], sum[1], sum[2], sum[3]);
+    *(float4 *)(p + 4) = make_float4(sum[4], sum[5], sum[6], sum[7]);
+}
+
+// out[c] = sum over b of part[b][c], fp32 or bf16: 32 columns per workgroup, kSumSlots threads a column,
+// in a fixed order.
+constexpr int kSumSlots = 16;
+__global__ __launch_bounds__(32 * kSumSlots) void k_colsum_reduce(const float *__restrict__ part, int blocks, int64_t cols,
+                                                         void *__restrict__ out, int f32)
+{
+    __shared__ float red[kSumSlots][33];
+    const int cc = threadIdx.x & 31, b0 = threadIdx.x >> 5;
+    const int64_t c = int64_t(blockIdx.x) * 32 + cc;
+    float a = 0.0f;
+    if (c < cols) {
+#pragma unroll 8
+        for (int b = b0; b < blocks; b += kSumSlots) a += part[int64_t(b) * cols + c];
+    }
+    red[b0][cc] = a;
+    __syncthreads();
+    if (b0 != 0 || c >= cols) return;
+#pragma unroll
+    for (int k = 1; k < kSumSlots; ++k) a += red[k][cc];
+    if (f32) ((float *)out)[c] = a;
+    else ((uint16_t *)out)[c] = uint16_t(f2bf(a));
 }
 
 // QFuncs/hif8.py:6-23 evaluated on a bf16 tensor without force_fp32 (quant_dequant_float with
@@ -1125,6 +1236,48 @@ int hif8_quantize_with_codes(const void *x, int dtype, int64_t n, float scale_ma
 {
     if (!codes || (dtype != HIF8_DTYPE_F32 && dtype != kBF16F32)) return HIF8_ERR_ARG;
     return quantize(x, dtype, n, scale_max, state, x_q, HIF8_OUT_BF16, HIF8_SEM_NPU, codes, stream);
+}
+
+// Rows per workgroup of k_quant_cols, a power of two: few enough to fill the chip (500 x 1536: 33 us with
+// 64 rows, 16 with 16), at most 4096 workgroups and 1024 partials of a column.
+static int colsum_rows(int64_t rows, int64_t strips)
+{
+    int64_t r = 16;
+    while (r < (1 << 20) && ((rows + r - 1) / r * strips > 4096 || (rows + r - 1) / r > 1024)) r *= 2;
+    return int(r);
+}
+static int64_t colsum_strips(int64_t cols) { return ((cols >> 3) + kTPB - 1) / kTPB; }
+
+int64_t hif8_quantize_colsum_workspace_bytes(int64_t rows, int64_t cols)
+{
+    if (rows <= 0 || cols <= 0) return 0;
+    const int64_t r = colsum_rows(rows, colsum_strips(cols));
+    return (rows + r - 1) / r * cols * 4;
+}
+
+int hif8_quantize_colsum(const uint16_t *x, int64_t rows, int64_t cols, float scale_max, void *state, uint16_t *x_q,
+                         void *colsum, int colsum_dtype, void *workspace, int64_t workspace_bytes,
+                         hif8_stream_t stream)
+{
+    if (!x || !state || !x_q || !colsum || !workspace || rows <= 0 || cols <= 0) return HIF8_ERR_ARG;
+    if (colsum_dtype != HIF8_DTYPE_BF16 && colsum_dtype != HIF8_DTYPE_F32) return HIF8_ERR_ARG;
+    if (cols % 8 != 0 || cols >= (int64_t(1) << 31) || rows >= (int64_t(1) << 31)) return HIF8_ERR_SHAPE;
+    if (!aligned16(x) || !aligned16(x_q) || !aligned16(workspace)) return HIF8_ERR_ALIGN;
+    if (workspace_bytes < hif8_quantize_colsum_workspace_bytes(rows, cols)) return HIF8_ERR_ARG;
+    const int64_t n = rows * cols, strips = colsum_strips(cols);
+    const int rpw = colsum_rows(rows, strips);
+    const int64_t blocks = (rows + rpw - 1) / rpw;
+    if (blocks >= 65536) return HIF8_ERR_SHAPE;
+    const int width = int(((cols >> 3) + strips - 1) / strips);
+    const int cap = cu_count() * kAmaxWgPerCu;
+    const int grid = grid_for((n + 63) / 64, cap < kMaxParts ? cap : kMaxParts);
+    hipStream_t s = (hipStream_t)stream;
+    hipLaunchKernelGGL((k_absmax<kBF16, true>), dim3(grid), dim3(kTPB), 0, s, x, n, (State *)state, scale_max);
+    hipLaunchKernelGGL(k_quant_cols, dim3(unsigned(strips), unsigned(blocks)), dim3(kTPB), 0, s, x, rows, cols,
+                       (State *)state, x_q, grid, scale_max, width, rpw, (float *)workspace);
+    hipLaunchKernelGGL(k_colsum_reduce, dim3(unsigned((cols + 31) / 32)), dim3(32 * kSumSlots), 0, s, (const float *)workspace,
+                       int(blocks), cols, colsum, colsum_dtype == HIF8_DTYPE_F32 ? 1 : 0);
+    return last_launch();
 }
 
 int hif8_encode(const void *x, int dtype, int64_t n, const void *state, uint8_t *codes, hif8_stream_t stream)

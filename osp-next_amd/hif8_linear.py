@@ -230,6 +230,28 @@ def quantize_with_codes(x: Tensor, scale_max: float) -> Tuple[Tensor, Tensor, Qu
     return xq, codes, st
 
 
+def quantize_colsum(x2: Tensor, scale_max: float, out_dtype: torch.dtype) -> Optional[Tuple[Tensor, Tensor]]:
+    """(x_q, x_q.sum(0) in ``out_dtype``) of a contiguous bf16 x [M, N] (hif8_quantize_colsum), or None
+    for shapes and dtypes it does not take."""
+    M, N = x2.shape
+    if (x2.dtype != torch.bfloat16 or N % 8 or M * N == 0 or out_dtype not in (torch.bfloat16, torch.float32)
+            or not x2.is_cuda):
+        return None
+    x2 = _aligned(x2)
+    L = _lib.load()
+    xq = torch.empty_like(x2)
+    sums = torch.empty(N, dtype=out_dtype, device=x2.device)
+    nbytes = int(L.hif8_quantize_colsum_workspace_bytes(M, N))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x2.device)
+    st = QuantState.unset(x2.device)
+    rc = L.hif8_quantize_colsum(x2.data_ptr(), M, N, float(scale_max), st.ptr, xq.data_ptr(), sums.data_ptr(),
+                                _lib.dtype_code(out_dtype), ws.data_ptr(), nbytes, _lib.stream_ptr(x2.device))
+    if rc == _lib.ERR_SHAPE:
+        return None
+    _lib.check(rc, "hif8_quantize_colsum")
+    return xq, sums
+
+
 def _quant(x: Tensor, scale_max: float, semantics: int = _lib.SEM_NPU) -> Tuple[Tensor, Tensor]:
     """hif8_linear.py:42-50: returns ``(x_q, scale)``, scale a 0-dim tensor of x's dtype."""
     xq, st = quantize(x.contiguous(), scale_max, _lib.OUT_SAME, semantics)
@@ -806,8 +828,15 @@ class _HIF8LinearFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         # x_q and w_q as the reference saves them (hif8_linear.py:78-82)
-        grad_q, _ = quantize(grad_output.contiguous(), ctx.smb)           # :93
-        g_2d = grad_q.reshape(-1, grad_q.shape[-1]).contiguous()
+        g_2d = grad_output.reshape(-1, grad_output.shape[-1]).contiguous()
+        grad_bias = None
+        with_sums = quantize_colsum(g_2d, ctx.smb, ctx.b_dtype) if ctx.has_bias else None
+        if with_sums is not None:                                         # :93 and :107 in one pass
+            g_2d, grad_bias = with_sums
+        else:
+            g_2d, _ = quantize(g_2d, ctx.smb)                             # :93
+            if ctx.has_bias:
+                grad_bias = g_2d.sum(0).to(ctx.b_dtype)                   # :107
         M, N = g_2d.shape
         K = ctx.packed.shape[1]
         g_bf16 = g_2d.dtype == torch.bfloat16
@@ -833,7 +862,6 @@ class _HIF8LinearFunction(torch.autograd.Function):
                 grad_weight = linear_wgrad(g_2d, x_2d).to(ctx.w_dtype)
             else:                                                         # g[M, N]^T x[M, K]
                 grad_weight = gemm_f32(g_2d, x_2d, N, K, M, (1, N), (K, 1)).to(ctx.w_dtype)
-        grad_bias = g_2d.sum(0).to(ctx.b_dtype) if ctx.has_bias else None                   # :107
         return grad_input, grad_weight, grad_bias, None, None, None, None
 
 
