@@ -358,8 +358,10 @@ int hif8_linear_wgrad_scaled(const uint16_t *g, const uint16_t *v, const void *v
 int hif8_linear_fwd_scaled(const uint16_t *a, const uint16_t *v, const void *v_state, void *y, int out_dtype,
                            int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes,
                            hif8_stream_t stream);
-/* The HiF8 values of codes, y = decode(code) in bf16 (exact); y 16-byte aligned. */
-int hif8_decode_values(const uint8_t *codes, int64_t n, uint16_t *y, hif8_stream_t stream);
+/* The HiF8 values of codes, y = decode(code) in bf16 (exact); y 16-byte aligned.  With the codes' state
+ * (null: none) a scale of 0 gives decode(code) / 0, so that a product divided by it afterwards is NaN
+ * where the product of the quotients is. */
+int hif8_decode_values(const uint8_t *codes, int64_t n, const void *state, uint16_t *y, hif8_stream_t stream);
 
 /* The backward's products for a layer that computes in fp32: grad_q @ w_q and grad_q^T @ x_q
  * (hif8_linear.py:97,104), which the reference evaluates as matmuls in the saved tensors' dtype.

@@ -50,7 +50,7 @@ SIGNATURES = {
     "hif8_linear_ksplit_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "hif8_linear_wgrad_scaled": (_i, [_p, _p, _p, _p, _i, _i64, _i64, _i64, _p, _i64, _p]),
     "hif8_linear_fwd_scaled": (_i, [_p, _p, _p, _p, _i, _i64, _i64, _i64, _p, _i64, _p]),
-    "hif8_decode_values": (_i, [_p, _i64, _p, _p]),
+    "hif8_decode_values": (_i, [_p, _i64, _p, _p, _p]),
     "hif8_linear_wgrad": (_i, [_p, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),
     "hif8_gemm_f32": (_i, [_p, _i, _p, _i, _p, _i, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p]),
     "hif8_pad_2d": (_i, [_p, _i64, _i64, _p, _i64, _i64, _i, _p]),

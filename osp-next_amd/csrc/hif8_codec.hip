@@ -263,6 +263,9 @@ __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int6
         float y;
         if (use_state) y = st->lut_f32[c];
         else y = u2f(decode_bits(c));
+        // HiF8 values for a product that is divided by the scale afterwards: a scale of 0 (an Inf in the
+        // tensor) makes 0 / 0 of the finite ones here, before the sums would hide it
+        if (MODE == 2 && !use_state && st && st->scale == 0.0f) y = y / st->scale;
         ((float *)(lds + kLdsLutF32))[c] = y;
         ((uint16_t *)(lds + kLdsLutBf16))[c] = use_state ? st->lut_bf16[c] : uint16_t(f2bf(y));
     }
@@ -1302,9 +1305,9 @@ int hif8_decode(const uint8_t *codes, int64_t n, const void *state, int out_dtyp
     return launch_quant(codes, out_dtype, n, state, y, 2, HIF8_SEM_NPU, 1, stream);
 }
 
-int hif8_decode_values(const uint8_t *codes, int64_t n, uint16_t *y, hif8_stream_t stream)
+int hif8_decode_values(const uint8_t *codes, int64_t n, const void *state, uint16_t *y, hif8_stream_t stream)
 {
-    return launch_quant(codes, HIF8_DTYPE_BF16, n, nullptr, y, 2, HIF8_SEM_NPU, 0, stream);
+    return launch_quant(codes, HIF8_DTYPE_BF16, n, state, y, 2, HIF8_SEM_NPU, 0, stream);
 }
 
 int hif8_quant_f32(const float *x, float *y, int64_t n, int semantics, hif8_stream_t stream)

@@ -414,13 +414,14 @@ def _ksplit_workspace(M: int, N: int, K: int, device: torch.device) -> Tuple[Opt
     return (torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=device) if nbytes > 0 else None), nbytes
 
 
-def decode_values(codes: Tensor) -> Tensor:
-    """The HiF8 values decode(code) of codes, exact in bf16 (hif8_decode_values)."""
+def decode_values(codes: Tensor, state: QuantState) -> Tensor:
+    """The HiF8 values decode(code) of codes, exact in bf16 (decode(code) / 0 where the state's scale is
+    0; hif8_decode_values)."""
     _lib.require_gpu_tensor(codes, "codes")
     codes = _aligned(codes)
     y = torch.empty(codes.shape, dtype=torch.bfloat16, device=codes.device)
     if codes.numel():
-        _lib.check(_lib.load().hif8_decode_values(codes.data_ptr(), codes.numel(), y.data_ptr(),
+        _lib.check(_lib.load().hif8_decode_values(codes.data_ptr(), codes.numel(), state.ptr, y.data_ptr(),
                                                   _lib.stream_ptr(codes.device)), "hif8_decode_values")
     return y
 
@@ -436,7 +437,7 @@ def linear_wgrad_scaled(grad_q2: Tensor, codes: Tensor, state: QuantState, out_d
     g = _aligned(pad_2d(grad_q2.contiguous(), M, Np) if Np != N else grad_q2.contiguous())
     if Kp != K:
         codes = pad_2d(codes.contiguous(), M, Kp)
-    v = decode_values(codes)
+    v = decode_values(codes, state)
     dw = torch.empty((Np, Kp), dtype=out_dtype, device=g.device)
     ws, nbytes = _ksplit_workspace(Np, Kp, M, g.device)
     rc = _lib.load().hif8_linear_wgrad_scaled(g.data_ptr(), v.data_ptr(), state.ptr, dw.data_ptr(),
@@ -460,7 +461,7 @@ def linear_dgrad_scaled(grad_q2: Tensor, w: "PackedWeight", out_dtype: torch.dty
     g = _aligned(grad_q2.contiguous())
     if Np != N:
         g = pad_2d(g, M, Np)
-    v = decode_values(w.codes_t() if (Np, Kp) == (N, K) else w.codes_t_padded(Kp, Np))
+    v = decode_values(w.codes_t() if (Np, Kp) == (N, K) else w.codes_t_padded(Kp, Np), w.state)
     y = torch.empty((M, Kp), dtype=out_dtype, device=g.device)
     ws, nbytes = _ksplit_workspace(M, Kp, Np, g.device)
     rc = _lib.load().hif8_linear_fwd_scaled(g.data_ptr(), v.data_ptr(), w.state.ptr, y.data_ptr(),

@@ -97,7 +97,9 @@ def test_wgrad_scaled_non_finite_input(pkg, value):
     got = pkg.hif8_linear.linear_wgrad_scaled(gq, codes, st, torch.float32)
     want = pkg.gemm_f32(gq, pkg.decode(codes, st, torch.float32), 64, 64, 130, (1, 64), (64, 1))
     assert not torch.isfinite(want).any()
-    assert not torch.isfinite(got).any()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    same = torch.isnan(want) | (got == want)
+    assert bool(same.all())
 
 
 @pytest.mark.gpu
@@ -152,4 +154,5 @@ def test_scaled_status_codes_without_gpu(pkg):
     assert wg(n=260) == -2 and wg(k=100) == -2 and wg(tokens=1 << 22) == -2 and wg(dw=fake + 2) == -3
     assert fw(a=None) == -1 and fw(dt=3) == -1 and fw(N=0) == -1
     assert fw(K=100) == -2 and fw(N=100) == -2 and fw(K=1 << 22) == -2 and fw(y=fake + 8) == -3
-    assert L.hif8_decode_values(None, 16, fake, None) == -1 and L.hif8_decode_values(fake, 16, fake + 4, None) == -3
+    assert L.hif8_decode_values(None, 16, None, fake, None) == -1
+    assert L.hif8_decode_values(fake, 16, None, fake + 4, None) == -3
