@@ -32,6 +32,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
 constexpr int kMaxChunks = 16;  // dim <= 8192
+constexpr int kAhead = 4;       // k_rms_norm_rope: the next row's loads a row ahead up to dim 2048
 
 __device__ __forceinline__ float lo(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
 __device__ __forceinline__ float hi(uint32_t v) { return __builtin_bit_cast(float, v & 0xFFFF0000u); }
@@ -46,7 +47,11 @@ __device__ __forceinline__ uint32_t pack(float a, float b) { return f2bf_pk(a, b
 // out = bf16 of that output's HiF8 fake quant with st's scale (the attention's bf16 cast of
 // _quant(q)), and y_out, if not null, the output itself (fp32 with rope, bf16 without).  For a
 // state with a finite scale the fake quant is the codec's table route (the encode table and the
-// state's bf16 decode table in LDS, fast_elem_bf16), otherwise the scalar route; the same bits.
+// state's bf16 decode table in LDS), a chunk's 8 elements at a time for the NPU semantics of a
+// finite tensor, else one by one (fast_elem_bf16); for other states the scalar route; the same bits.
+// Bound by that arithmetic and the latency of a row's chain.  Rope forms, us, amax / fake quant
+// ([34944, 1536] over 8736 positions; [32760, 5120]): 64-bit row quotients, no loads ahead, element
+// by element 30 / 53; 86 / 229.  Now 27 / 42 (5.1 TB/s); 81 / 142 (4.7 TB/s).
 template <int NC, bool ROPE, int MODE>
 __global__ __launch_bounds__(kThreads) void k_rms_norm_rope(const uint16_t *__restrict__ x, const float *__restrict__ w,
                                                             const float *__restrict__ cs, const float *__restrict__ sn,
@@ -63,6 +68,7 @@ __global__ __launch_bounds__(kThreads) void k_rms_norm_rope(const uint16_t *__re
     __shared__ __attribute__((aligned(16))) uint8_t qtab[MODE == 2 ? kLdsBytes : 16];
     const bool qfast = MODE == 2 && st->fast != 0;
     const bool nan_guard = MODE == 2 && st->finite == 0;
+    const bool qplain = qfast && !nan_guard && sem == kSemNpu;
     if (MODE == 2) {
         if (qfast) {
             ((uint16_t *)(qtab + kLdsLutBf16))[threadIdx.x] = st->lut_bf16[threadIdx.x];
@@ -74,11 +80,41 @@ __global__ __launch_bounds__(kThreads) void k_rms_norm_rope(const uint16_t *__re
     }
     const int64_t wstride = int64_t(gridDim.x) * (kThreads / 64);
     const float inv_dim = 1.0f / float(dim);
-    for (int64_t row = int64_t(blockIdx.x) * (kThreads / 64) + (threadIdx.x >> 6); row < rows; row += wstride) {
-        const u32x4 *xr = (const u32x4 *)(x + row * dim);
-        u32x4 v[NC];
+    const int64_t row0 = int64_t(blockIdx.x) * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // A row is one chain of load, reduction and store.  Short rows (up to kAhead chunks a lane) keep the
+    // next row's loads in flight over it; longer ones have enough of their own.  The rope row's quotients
+    // are 32-bit where the row count allows (three 64-bit divisions cost as much as a 1536-wide row).
+    constexpr bool kPre = NC <= kAhead;
+    u32x4 nv[NC] = {};
+    if (kPre && row0 < rows) {
+        const u32x4 *xr = (const u32x4 *)(x + row0 * dim);
 #pragma unroll
-        for (int c = 0; c < NC; ++c) v[c] = __builtin_nontemporal_load(&xr[c * 64 + lane]);
+        for (int c = 0; c < NC; ++c) nv[c] = __builtin_nontemporal_load(&xr[c * 64 + lane]);
+    }
+    for (int64_t row = row0; row < rows; row += wstride) {
+        f32x4 ca = {}, sa = {};
+        if (ROPE) {
+            int64_t cr;
+            if (rows <= int64_t(0x7FFFFFFF)) {   // seq divides rows; rep may be larger
+                const uint32_t q = uint32_t(row) / uint32_t(seq), s = uint32_t(row) - q * uint32_t(seq);
+                cr = (rep <= int64_t(0x7FFFFFFF) ? int64_t(q / uint32_t(rep)) : 0) * seq + s;
+            } else {
+                cr = (row / seq / rep) * seq + row % seq;
+            }
+            const int pair = ((lane * 8) % head_dim) / 2;
+            const int d = head_dim / 2;
+            ca = *(const f32x4 *)(cs + cr * d + pair);
+            sa = *(const f32x4 *)(sn + cr * d + pair);
+        }
+        u32x4 v[NC];
+        const int64_t next = kPre ? row + wstride : row;
+        const u32x4 *xr = (const u32x4 *)(x + next * dim);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[c] = nv[c];
+        if (next < rows) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) (kPre ? nv : v)[c] = __builtin_nontemporal_load(&xr[c * 64 + lane]);
+        }
         float ss = 0.f;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
@@ -92,15 +128,6 @@ __global__ __launch_bounds__(kThreads) void k_rms_norm_rope(const uint16_t *__re
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
         const float r = rsqrtf(ss * inv_dim + eps);
-        f32x4 ca = {}, sa = {};
-        if (ROPE) {
-            const int64_t s = row % seq;
-            const int64_t cr = (row / seq / rep) * seq + s;
-            const int pair = ((lane * 8) % head_dim) / 2;
-            const int d = head_dim / 2;
-            ca = *(const f32x4 *)(cs + cr * d + pair);
-            sa = *(const f32x4 *)(sn + cr * d + pair);
-        }
         u32x4 *orow = (u32x4 *)(out + row * dim);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
@@ -148,24 +175,56 @@ __global__ __launch_bounds__(kThreads) void k_rms_norm_rope(const uint16_t *__re
                     amax = m > amax ? m : amax;
                 }
             } else {
-                uint32_t qb[8];
+                u32x4 q;
+                if (qplain) {
+                    // all of a chunk's code lookups in flight together, then all of its decode lookups
+                    uint32_t t16[8];   // the bf16 bits (fp32: truncated) of y * s
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    if (qfast) {
-                        qb[e] = fast_elem_bf16<ROPE ? kF32 : kBF16>(f[e], qs, sem, qtab, nan_guard);
-                    } else {
-                        uint32_t yb, code;
+                    for (int e = 0; e < 8; e += 2) {
                         if (ROPE) {
-                            slow_elem<kF32>(__builtin_bit_cast(uint32_t, f[e]), qs, sem, yb, code);
-                            qb[e] = f2bf(u2f(yb));
+                            t16[e] = __builtin_bit_cast(uint32_t, f[e] * qs) >> 16;
+                            t16[e + 1] = __builtin_bit_cast(uint32_t, f[e + 1] * qs) >> 16;
                         } else {
-                            slow_elem<kBF16>(__builtin_bit_cast(uint32_t, f[e]) >> 16, qs, sem, yb, code);
-                            qb[e] = yb;
+                            const uint32_t p = pack(f[e] * qs, f[e + 1] * qs);
+                            t16[e] = p & 0xFFFFu;
+                            t16[e + 1] = p >> 16;
                         }
                     }
+                    const uint16_t *lut16 = (const uint16_t *)(qtab + kLdsLutBf16);
+                    uint32_t code[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const uint32_t *t = t16 + 4 * h;
+                        const uint32_t mags = uint32_t(qtab[clampu(t[0] & 0x7FFFu)]) | (uint32_t(qtab[clampu(t[1] & 0x7FFFu)]) << 8) |
+                                              (uint32_t(qtab[clampu(t[2] & 0x7FFFu)]) << 16) | (uint32_t(qtab[clampu(t[3] & 0x7FFFu)]) << 24);
+                        code[h] = apply_signs(mags, ((t[0] & 0x8000u) >> 8) | (t[1] & 0x8000u) | ((t[2] & 0x8000u) << 8) |
+                                                        ((t[3] & 0x8000u) << 16));
+                    }
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const uint32_t d = code[t >> 1] >> (16 * (t & 1));
+                        q[t] = uint32_t(lut16[d & 0xFFu]) | (uint32_t(lut16[(d >> 8) & 0xFFu]) << 16);
+                    }
+                } else {
+                    uint32_t qb[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        if (qfast) {
+                            qb[e] = fast_elem_bf16<ROPE ? kF32 : kBF16>(f[e], qs, sem, qtab, nan_guard);
+                        } else {
+                            uint32_t yb, code;
+                            if (ROPE) {
+                                slow_elem<kF32>(__builtin_bit_cast(uint32_t, f[e]), qs, sem, yb, code);
+                                qb[e] = f2bf(u2f(yb));
+                            } else {
+                                slow_elem<kBF16>(__builtin_bit_cast(uint32_t, f[e]) >> 16, qs, sem, yb, code);
+                                qb[e] = yb;
+                            }
+                        }
+                    }
+                    q = u32x4{qb[0] | (qb[1] << 16), qb[2] | (qb[3] << 16), qb[4] | (qb[5] << 16), qb[6] | (qb[7] << 16)};
                 }
-                orow[c * 64 + lane] = u32x4{qb[0] | (qb[1] << 16), qb[2] | (qb[3] << 16), qb[4] | (qb[5] << 16),
-                                            qb[6] | (qb[7] << 16)};
+                orow[c * 64 + lane] = q;
                 if (y_out) {
                     if (ROPE) {
                         f32x4 *yr = (f32x4 *)((float *)y_out + row * dim + c * 512 + lane * 8);
