@@ -96,7 +96,8 @@ int hif8_set_scale(void *state, int dtype, float scale, hif8_stream_t stream);
  * workgroups' maxima in state, which need not be initialised, and the quantisation pass reduces them
  * and settles state as hif8_absmax_scale would (the reference's _quant, hif8_linear.py:42-50).
  * out_kind HIF8_OUT_CODES: hif8_encode's codes (semantics HIF8_SEM_NPU); HIF8_OUT_SAME: hif8_fake_quant's
- * x_q; HIF8_OUT_BF16: hif8_fake_quant_to_bf16's; the same bytes as those entry points give.  x and out
+ * x_q (fp32, 4 n bytes, for HIF8_DTYPE_F32 and HIF8_DTYPE_BF16_AS_F32); HIF8_OUT_BF16:
+ * hif8_fake_quant_to_bf16's; the same bytes as those entry points give.  x and out
  * 16-byte aligned, n > 0. */
 #define HIF8_OUT_CODES 0
 #define HIF8_OUT_SAME 1

@@ -198,7 +198,7 @@ def quantize(x: Tensor, scale_max: float, out_kind: int = _lib.OUT_SAME, semanti
              as_f32: bool = False) -> Tuple[Tensor, QuantState]:
     """``absmax_scale`` into a fresh state, then ``encode`` (OUT_CODES), ``fake_quant`` (OUT_SAME) or
     ``fake_quant_to_bf16`` (OUT_BF16) of a contiguous x, in two launches (hif8_quantize): the same bytes
-    and state."""
+    and state.  OUT_SAME with ``as_f32`` gives the fp32 x_q of ``x.float()``."""
     _lib.require_gpu_tensor(x, "x")
     x = _aligned(x)
     n = x.numel()
@@ -206,7 +206,7 @@ def quantize(x: Tensor, scale_max: float, out_kind: int = _lib.OUT_SAME, semanti
         raise ValueError("amax of an empty tensor")
     dtype = _dtype_arg(x, as_f32)
     if out_kind == _lib.OUT_SAME:
-        out = torch.empty_like(x)
+        out = torch.empty_like(x, dtype=torch.float32 if as_f32 else None)
     else:
         out = torch.empty(x.shape, dtype=torch.uint8 if out_kind == _lib.OUT_CODES else torch.bfloat16, device=x.device)
     st = QuantState.unset(x.device)

@@ -69,8 +69,34 @@ def test_degenerate_scales(pkg, special, dtype):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1000, SPAN + 48])
 def test_bf16_as_f32(pkg, n):
+    x = inputs(n, torch.bfloat16, None, 3)
     for kind in (0, 3):
-        both(pkg, inputs(n, torch.bfloat16, None, 3), kind, 0, as_f32=True)
+        both(pkg, x, kind, 0, as_f32=True)
+    got, st = pkg.hif8_linear.quantize(x, 15.0, as_f32=True)      # OUT_SAME: the fp32 x_q of x.float()
+    want, ref = pkg.hif8_linear.quantize(x.float(), 15.0)
+    assert got.dtype == torch.float32 and torch.equal(got, want) and st.read() == ref.read()
+
+
+@pytest.mark.parametrize("dtype,as_f32", [("bfloat16", False), ("float32", False), ("bfloat16", True)])
+@pytest.mark.parametrize("kind", [0, 1, 3])
+def test_output_holds_what_the_kernel_writes(pkg, monkeypatch, dtype, as_f32, kind):
+    """quantize allocates the bytes that hif8_quantize writes for its dtype and kind (hif8_mi355x.h): codes
+    1 an element, OUT_BF16 2, OUT_SAME 2 for a bf16 tensor and 4 for fp32 arithmetic, bf16 storage or not."""
+    lib, calls = pkg._lib, []
+
+    class Recorder:
+        def hif8_quantize(self, *args):
+            calls.append(args)
+            return 0
+    monkeypatch.setattr(lib, "load", Recorder)
+    monkeypatch.setattr(lib, "require_gpu_tensor", lambda t, name: None)
+    monkeypatch.setattr(lib, "stream_ptr", lambda device: 0)
+    monkeypatch.setattr(lib, "unset_state", lambda device: torch.empty(4096, dtype=torch.uint8))
+    x = torch.zeros(5, 32, dtype=getattr(torch, dtype))
+    out, _ = pkg.hif8_linear.quantize(x, 15.0, kind, as_f32=as_f32)
+    (_, code, n, _, _, ptr, _, _, _), = calls
+    writes = {0: 1, 3: 2, 1: 2 if code == lib.DTYPE_BF16 else 4}[kind]
+    assert ptr == out.data_ptr() and n == x.numel() and out.element_size() == writes and out.shape == x.shape
 
 
 @pytest.mark.gpu
