@@ -115,7 +115,10 @@ def check(status: int, what: str) -> None:
 
 
 def stream_ptr(device: torch.device) -> int:
-    """The current stream's handle, without building a Stream object (four or more times a linear)."""
+    """The current stream's handle on a GPU, without building a Stream object (four or more times a
+    linear).  Refuses other devices: a launch would take their pointers as the GPU's."""
+    if device.type != "cuda":
+        raise ValueError(f"the HiF8 path has no CPU route: expected a GPU device, got {device}")
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 

@@ -199,6 +199,30 @@ def test_python_layer_refuses_cpu_tensors(pkg):
         pkg.key_list(torch.ones(2, 3))          # not a bool mask
 
 
+def test_host_memory_never_reaches_a_launch(pkg, monkeypatch):
+    """Calls without a check of their own take their stream from their tensor's device, which must be a
+    GPU's: no library function is called with host pointers, whatever GPU is current."""
+    torch = pytest.importorskip("torch")
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0, raising=False)
+
+    class Recorder:
+        def __getattr__(self, name):
+            def launch(*args):
+                assert name.endswith(("_size", "_bytes")), f"{name} was called"
+                return 4096
+            return launch
+    monkeypatch.setattr(pkg._lib, "load", Recorder)
+    for device in ("cpu", "meta"):
+        with pytest.raises(ValueError):
+            pkg._lib.stream_ptr(torch.device(device))
+    a, w = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(8, 64, dtype=torch.bfloat16)
+    for call in (lambda: pkg.QuantState("cpu"), lambda: pkg.linear_fwd_wq(a, w, None),
+                 lambda: pkg.hif8_linear.linear_fwd_wq_split(a, w), lambda: pkg.linear_wgrad(a, a)):
+        with pytest.raises(ValueError):
+            call()
+
+
 @pytest.fixture(scope="module")
 def hostlib(tmp_path_factory):
     out = tmp_path_factory.mktemp("hostchk") / "libhostchk.so"
