@@ -493,7 +493,8 @@ int hif8_ln_affine_fake_quant(const uint16_t *x, const float *weight, const floa
  * key_idx NULL and key_count NULL: every key 0 .. n_kv - 1.  key_count [batch] alone: the first
  * key_count[b] keys.  key_idx [batch][idx_batch_stride] with key_count: the key rows
  * key_idx[b][0 .. key_count[b] - 1] (entries clamped to [0, n_kv)).  A query with no key gets
- * zeros (the reference raises for a sequence whose keys are all masked).
+ * zeros (the reference raises for a sequence whose keys are all masked); one whose kept keys' scores
+ * are all -inf gets NaN, as softmax gives, and keys of score -inf beside finite ones count nothing.
  * row_strides and batch_strides are host arrays of 4.
  * out_state NULL: attention only.  Otherwise the o projection's input state: the kernel folds the
  * amax of out and a one-workgroup kernel after it writes amax, scale (rule for scale_max) and

@@ -68,7 +68,7 @@ constexpr int kBM = kWaves * kQW;        // queries per workgroup
 constexpr uint32_t kTile = kBN * kD * 2;  // bytes of one K or V tile
 constexpr uint32_t kList = 4 * kTile;     // key-list ring: 3 slots of one tile's 64 entries
 constexpr uint32_t kLds = kList + 3 * kBN * 4;
-constexpr float kNoKey = -3.0e38f;        // reference max before any key
+constexpr float kNoKey = -3.40282347e38f; // reference max while every score is -inf
 constexpr float kLazy = 8.0f;             // log2 headroom before the reference max moves
 
 struct Params {
@@ -86,6 +86,27 @@ struct Params {
     int full, splits;                // query tiles [0, full) whole, the others in `splits` key ranges
     float *part;                     // the ranges' partials (kPart floats each)
 };
+
+// The keys batch b uses.
+__device__ __forceinline__ int keys_of(const Params &p, int b)
+{
+    int nk = p.n_kv;
+    if (p.key_count) {
+        nk = p.key_count[b];
+        nk = nk < 0 ? 0 : (nk > p.n_kv ? p.n_kv : nk);
+        if (p.key_idx && int64_t(nk) > p.idx_bs) nk = int(p.idx_bs);
+    }
+    return nk;
+}
+
+// What a query's sums are multiplied by: 1 / l; without keys 0; NaN, softmax's value, where every score of
+// its keys is -inf and the reference maximum m never moved (an Inf in q or k, or an overflowed product,
+// must not pass for a zero output).
+__device__ __forceinline__ float out_factor(float l, float m, int nk)
+{
+    if (nk > 0 && m == kNoKey) return __builtin_nanf("");
+    return l > 0.f ? 1.0f / l : 0.f;
+}
 
 // One key range of one query tile: the waves' O accumulators unscaled, 1 KB per store instruction
 // ([wave][qb][d][lane] f32x4), then each query's reference max (log2) and sum ([2][wave][qb][16]).
@@ -184,13 +205,7 @@ template <bool LIST, bool SPLIT> __global__ __launch_bounds__(kThreads, 1) void 
     const int qt = L % p.q_tiles, bh = L / p.q_tiles;
     const int h = bh % p.heads, b = bh / p.heads;
 
-    int nk = p.n_kv;
-    if (p.key_count) {
-        nk = p.key_count[b];
-        nk = nk < 0 ? 0 : (nk > p.n_kv ? p.n_kv : nk);
-        if (p.key_idx && int64_t(nk) > p.idx_bs) nk = int(p.idx_bs);
-    }
-    nk = __builtin_amdgcn_readfirstlane(nk);
+    const int nk = __builtin_amdgcn_readfirstlane(keys_of(p, b));
     int t0 = 0, ntiles = (nk + kBN - 1) / kBN;   // this workgroup's key tiles: t0 .. ntiles - 1
     if (split) {
         const int len = (ntiles + p.splits - 1) / p.splits;
@@ -313,7 +328,7 @@ template <bool LIST, bool SPLIT> __global__ __launch_bounds__(kThreads, 1) void 
 #pragma unroll
     for (int d = 0; d < 8; ++d)
         o[d][0] = o[d][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // below every score, and finite: keys whose scores are all -inf get probabilities 0
+    // below every score, and finite: a tile whose scores are all -inf adds probabilities 0
     float mref[2] = {kNoKey, kNoKey};
     float lsum[2] = {0.f, 0.f};
     const float c = p.c;
@@ -443,7 +458,7 @@ template <bool LIST, bool SPLIT> __global__ __launch_bounds__(kThreads, 1) void 
         float l = lsum[qb];
         l += __shfl_xor(l, 16, 64);
         l += __shfl_xor(l, 32, 64);
-        const float inv = l > 0.f ? 1.0f / l : 0.f;
+        const float inv = out_factor(l, mref[qb], nk);
         const int row = qbase + 16 * qb + int(cq);
         if (row < p.n_q) {
             uint16_t *orow = p.out + int64_t(b) * p.o_bs + int64_t(row) * p.o_rs + int64_t(h) * kD + 4 * g;
@@ -502,7 +517,7 @@ __global__ __launch_bounds__(256) void k_attn_combine(const Params p)
         o0 += a * po[0];
         o1 += a * po[64];
     }
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const float inv = out_factor(l, m, keys_of(p, b));
     const int row = qt * kBM + int(wave) * kQW + int(qb) * 16 + int(cq);
     uint32_t amax = 0;
     if (row < p.n_q) {

@@ -31,7 +31,7 @@ def reference(q, k, v, rows):
     return out
 
 
-def unsplit(pkg, q, k, v, idx, cnt):
+def unsplit(pkg, q, k, v, idx, cnt, state=None):
     B, Nq, H, _ = q.shape
     out = torch.empty_like(q)
     I4 = ctypes.c_int64 * 4
@@ -40,7 +40,7 @@ def unsplit(pkg, q, k, v, idx, cnt):
     pkg._lib.check(pkg._lib.load().hif8_attention_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, Nq, k.shape[1], H, D, rs, bs,
         idx.data_ptr() if idx is not None else None, idx.stride(0) if idx is not None else 0,
-        cnt.data_ptr() if cnt is not None else None, 1.0 / math.sqrt(D), None, 2, 15.0,
+        cnt.data_ptr() if cnt is not None else None, 1.0 / math.sqrt(D), state.ptr if state else None, 2, 15.0,
         pkg._lib.stream_ptr(q.device)), "hif8_attention_fwd")
     return out
 
@@ -104,6 +104,41 @@ def test_key_ranges_nan(pkg):
     out = pkg.attention_fwd(q, k, v)
     bad = torch.isnan(out.float()).any(-1).squeeze()
     assert bad[33] and int(bad.sum()) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("split", [True, False])
+def test_infinite_scores(pkg, split):
+    """Keys of score -inf add nothing beside finite ones, also where they fill whole key tiles or a whole
+    key range; where all of a query's keys score -inf its output is NaN (float64 softmax's), and so is the
+    o state's amax; without keys it is zero."""
+    B, Nq, Nkv, H = 2, 300, 1200, 2
+    assert pkg._lib.load().hif8_attention_workspace_bytes(B, Nq, Nkv, H) > 0
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(B, n, H, D, generator=g).to(torch.bfloat16).to(DEV) for n in (Nq, Nkv, Nkv))
+    q[..., 7] = q[..., 7].abs() + 0.25
+    rows = [torch.arange(Nkv, device=DEV)] * B
+
+    def run(k, cnt=None):
+        st = pkg.QuantState(DEV)
+        out = (pkg.attention_fwd(q, k, v, None, cnt, o_state=st, o_as_f32=True) if split
+               else unsplit(pkg, q, k, v, None, cnt, st))
+        assert st.read()[0] == pkg.absmax_scale(out, 15.0, pkg.QuantState(DEV), True).read()[0]
+        return out
+    some = k.clone()
+    some[0, :700, :, 7] = float("-inf")           # the first tiles and ranges of batch 0
+    some[1, 640:704, :, 7] = float("-inf")        # one key tile of batch 1
+    ref = reference(q, some, v, rows)
+    err = (run(some).double() - ref).abs()
+    assert float(err.max()) <= 2e-2 * float(ref.abs().max()) and float(err.norm()) <= 1e-2 * float(ref.norm())
+    every = k.clone()
+    every[1, :, :, 7] = float("-inf")
+    out = run(every)
+    assert bool(torch.isnan(reference(q, every, v, rows)[1]).all())
+    assert bool(torch.isnan(out[1]).all()) and bool(torch.isfinite(out[0]).all())
+    cnt = torch.tensor([0, 5], dtype=torch.int32, device=DEV)
+    out = run(every, cnt)
+    assert bool((out[0] == 0).all()) and bool(torch.isnan(out[1]).all())
 
 
 def test_attention_plan_on_256_cus(pkg):
