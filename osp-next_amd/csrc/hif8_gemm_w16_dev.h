@@ -201,13 +201,20 @@ template <int SET, bool TR> __device__ __forceinline__ void tie_set(Ctx<TR> &c)
 
 #include "hif8_gemm_schedule_w16.inc"
 
-// a / s as IEEE division gives it: the product with the rounded reciprocal, corrected by its exact
-// remainder (two fma); where the quotient is not finite the correction would turn an infinity into NaN.
+// a / s for a scale s >= 0, Inf or NaN: the product with the rounded reciprocal, corrected by its exact
+// remainder (two fma), the IEEE quotient wherever that is a normal number.  Below 2^-126, where the
+// reciprocal may overflow (an fp32 tensor with an amax above scale_max * 2^126), a and s are both taken
+// 2^64 times: a sum that overflows so has an infinite quotient.  Where the quotient is not finite the
+// correction would turn an infinity into NaN; an infinite s leaves none (the quotient is 0).
 struct Divisor {
-    float s, r;
-    __device__ explicit Divisor(float scale) : s(scale), r(1.0f / scale) {}
+    float up, s, r;
+    __device__ explicit Divisor(float scale) : up(scale < 0x1p-126f ? 0x1p64f : 1.0f), s(scale * up), r(1.0f / s)
+    {
+        if (s == __builtin_inff()) s = 0.0f;
+    }
     __device__ __forceinline__ float operator()(float a) const
     {
+        a *= up;
         const float q = a * r;
         const float c = __builtin_fmaf(__builtin_fmaf(-q, s, a), r, q);
         return __builtin_fabsf(q) < __builtin_inff() ? c : q;

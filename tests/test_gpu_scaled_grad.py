@@ -103,6 +103,31 @@ def test_wgrad_scaled_non_finite_input(pkg, value):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(130, 64, 64), (2100, 1536, 1536)])   # whole tiles, k ranges
+def test_scale_with_overflowing_reciprocal(pkg, M, N, K):
+    """An fp32 operand of amax 1e38 under a scale_max of 0.1 has a scale of 1e-39, whose reciprocal is
+    infinite: the quotients, zero sums among them, are those of the decoded operand."""
+    gen = torch.Generator().manual_seed(M)
+    gq = (torch.randn(M, N, generator=gen) * 2.0 ** -10).to(torch.bfloat16).to(DEV)
+    x = torch.randn(M, K, generator=gen).clamp(-3, 3) * 2e37
+    x[:, 3] = 0
+    x[5, 7] = 1e38
+    x = x.to(DEV)
+    st = pkg.absmax_scale(x, 0.1, pkg.QuantState(DEV))
+    assert 0 < st.read()[1] < 2.0 ** -128
+    codes = pkg.encode(x, st)
+    for out_dtype in (torch.float32, torch.bfloat16):
+        got = pkg.hif8_linear.linear_wgrad_scaled(gq, codes, st, out_dtype)
+        bound(got, gq.t().contiguous(), pkg.decode(codes, st, torch.float32), out_dtype)
+        assert bool((got[:, 3] == 0).all())
+    packed = pkg.PackedWeight(x[:N].contiguous(), 0.1)
+    g = gq[:, :packed.shape[0]].contiguous()
+    if packed.shape[0] % 64 == 0:
+        bound(pkg.hif8_linear.linear_dgrad_scaled(g, packed, torch.float32), g, packed.dequantize(torch.float32),
+              torch.float32)
+
+
+@pytest.mark.gpu
 def test_wgrad_small_grid_split(pkg):
     """36 tiles over 4100 tokens run as k ranges: bounded against float64, equal to the transposed
     route bit for bit, and the same on a second call."""
