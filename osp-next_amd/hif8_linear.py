@@ -344,8 +344,10 @@ def linear_dgrad(grad_q2: Tensor, w: "PackedWeight", out_dtype: torch.dtype = to
         w_qt = decode(codes_t, w.state, torch.bfloat16)
         if out_dtype == torch.float32:
             y = torch.empty((M, Kp), dtype=torch.float32, device=g.device)
+            ws, nbytes = _ksplit_workspace(M, Kp, Np, g.device)
             _lib.check(_lib.load().hif8_linear_fwd_scaled(g.data_ptr(), w_qt.data_ptr(), None, y.data_ptr(),
-                                                          _lib.DTYPE_F32, M, Kp, Np, None, 0,
+                                                          _lib.DTYPE_F32, M, Kp, Np,
+                                                          ws.data_ptr() if ws is not None else None, nbytes,
                                                           _lib.stream_ptr(g.device)), "hif8_linear_fwd_scaled")
         else:
             y = linear_fwd_wq_split(g, w_qt)

@@ -73,7 +73,7 @@ def test_dgrad_scaled(pkg, M, N, K, out_dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(8192, 2112, 40), (8200, 2304, 264), (24600, 64, 8), (8193, 2100, 36)])
+@pytest.mark.parametrize("M,N,K", [(8192, 2112, 40), (8200, 2304, 264), (24600, 64, 8), (8193, 2100, 36), (8192, 2112, 2304)])
 def test_dgrad_fp32_output(pkg, M, N, K):
     """The gradient of an fp32 input with a bf16 weight on the decode-once route: fp32, unrounded."""
     print(f"[scaled] dgrad fp32 M={M} N={N} K={K}", flush=True)
@@ -164,6 +164,51 @@ def test_ksplit_plan_on_256_cus(pkg):
             sp = parts // tail
             per = -(-nk // sp)
             assert (sp - 1) * per < nk and nk >= 8 * sp
+
+
+class Calls:
+    """The library with its launches recorded instead of made (its size queries answered by itself)."""
+
+    def __init__(self, lib):
+        self.lib, self.made = lib, {}
+
+    def __getattr__(self, name):
+        if name.endswith(("_bytes", "_size")):
+            return getattr(self.lib, name)
+
+        def launch(*args):
+            self.made[name] = args
+            return 0
+        return launch
+
+
+def dgrad_calls(pkg, monkeypatch, M, N, K, out_dtype):
+    """The launches of linear_dgrad for a bf16 gradient [M, N] and a bf16 weight [N, K]."""
+    calls = Calls(pkg._lib.load())
+    monkeypatch.setattr(pkg._lib, "load", lambda: calls)
+    monkeypatch.setattr(pkg._lib, "stream_ptr", lambda device: 0)
+    monkeypatch.setattr(pkg._lib, "require_gpu_tensor", lambda t, name: None)
+
+    class Packed:
+        shape = (N, K)
+
+        class state:
+            ptr = 1
+
+        def codes_t(self):
+            return torch.empty(K, N, dtype=torch.uint8)
+    y = pkg.linear_dgrad(torch.empty(M, N, dtype=torch.bfloat16), Packed(), out_dtype)
+    assert y.dtype == out_dtype and y.shape == (M, K)
+    return calls.made
+
+
+@pytest.mark.parametrize("M,N,K", [(8192, 2112, 2304), (8192, 2112, 256)])
+def test_dgrad_fp32_output_splits(pkg, monkeypatch, M, N, K):
+    """The fp32 input gradient on the decode-once route gets the partials of its k ranges, on grids with a
+    short last wave (288 tiles) and below one wave (32 tiles)."""
+    want = pkg._lib.load().hif8_linear_ksplit_workspace_bytes(M, K, N)
+    made = dgrad_calls(pkg, monkeypatch, M, N, K, torch.float32)
+    assert want > 0 and made["hif8_linear_fwd_scaled"][-2] == want
 
 
 def test_scaled_status_codes_without_gpu(pkg):
