@@ -197,6 +197,10 @@ int hif8_quant_f16(const uint16_t *x, uint16_t *y, int64_t n, int semantics, hif
  */
 int hif8_linear_fwd(const uint16_t *a, const uint8_t *w_codes, const void *w_state, const uint16_t *bias,
                     uint16_t *y, int64_t M, int64_t N, int64_t K, hif8_stream_t stream);
+/* The same product without a bias and with the fp32 sums as the output, y: [M,N] row-major fp32 (the input
+ * gradient grad_q @ w_q of hif8_linear.py:97 for an fp32 input, with the transposed weight codes). */
+int hif8_linear_fwd_f32(const uint16_t *a, const uint8_t *w_codes, const void *w_state, float *y, int64_t M, int64_t N,
+                        int64_t K, hif8_stream_t stream);
 
 /* Several HIF8Linear layers on the same quantised input in one launch: the self-attention
  * q, k, v projections of osp_next.py:742-744 (each an F.linear(x_q, w_q, b) of

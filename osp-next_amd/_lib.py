@@ -43,6 +43,7 @@ SIGNATURES = {
     "hif8_quant_bf16": (_i, [_p, _p, _i64, _i, _p]),
     "hif8_quant_f16": (_i, [_p, _p, _i64, _i, _p]),
     "hif8_linear_fwd": (_i, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p]),
+    "hif8_linear_fwd_f32": (_i, [_p, _p, _p, _p, _i64, _i64, _i64, _p]),
     "hif8_transpose_codes": (_i, [_p, _i64, _i64, _p, _p]),
     "hif8_transpose_bf16": (_i, [_p, _i64, _i64, _i64, _p, _p]),
     "hif8_linear_split_workspace_bytes": (_i64, [_i64, _i64, _i64]),

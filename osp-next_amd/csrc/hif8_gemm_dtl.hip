@@ -227,13 +227,15 @@ __device__ __forceinline__ void tie_cd(Ctx &c)
 // accumulator; the settle kernel launched after it writes amax|GELU(y)| and its scale when max y
 // settles them, so that the down-projection's quantisation, which applies GELU, needs no amax
 // pass of its own (hif8_gelu_dev.h).
+// EPI 0 with f32: y = acc in fp32, no bias (the gradient of an fp32 input, which would otherwise be
+// rounded to bf16 and widened by a pass of its own), one output group.
 // The output features are G.n groups (G.n = 1 for one linear): the tile's group supplies its
 // decode table and its output buffer.
 template <int EPI>
 __global__ __launch_bounds__(kThreads, 1) void k_linear_dtl(const uint16_t *__restrict__ X, const uint8_t *__restrict__ Wc,
                                                             const Groups G, const uint16_t *__restrict__ bias,
                                                             int M, int N, int K, int tiles_m, int tiles_n,
-                                                            State *__restrict__ y_st)
+                                                            State *__restrict__ y_st, int f32)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[kLds];
     ASMV("; lds base %0" ::"v"(uint32_t(uintptr_t(smem))) : "memory");
@@ -400,6 +402,23 @@ __global__ __launch_bounds__(kThreads, 1) void k_linear_dtl(const uint16_t *__re
 #pragma unroll
         for (int j = 0; j < 16; ++j) ASMV("" : "+a"(c.acc[i][j]));
 
+    if (EPI == 0 && f32) {
+        // straight from the accumulators: 4 consecutive features, 16 bytes, per lane.  (Either way out ties
+        // each accumulator to its AGPRs where it uses it: without that all of them were copied to VGPRs
+        // ahead of the branch and spilled.)
+        float *Yf = (float *)Y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int n = n0 + int(c.wave * 64u + uint32_t(i * 16) + 4u * g);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int m = m0 + j * 16 + int(r);
+                ASMV("" : "+a"(c.acc[i][j]));
+                if (m < M && n < N) *(f32x4 *)(Yf + size_t(m) * size_t(N) + size_t(n)) = c.acc[i][j];
+            }
+        }
+        return;
+    }
     // Epilogue.  acc[i][j] lane (r, g), element e: D[n][m] with n = 64w + 16i + 4g + e,
     // m = 16j + r.  Rows go to LDS (padded), then each wave stores 2 rows x 512 B per instruction.
     __syncthreads();
@@ -416,6 +435,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_linear_dtl(const uint16_t *__re
                 const float b3 = __builtin_bit_cast(float, bb.y & 0xFFFF0000u);
 #pragma unroll
                 for (int j = 0; j < 16; ++j) {
+                    ASMV("" : "+a"(c.acc[i][j]));
                     const f32x4 &a = c.acc[i][j];
                     uint2 v;
                     v.x = f2bf_pk(a[0] + b0, a[1] + b1);
@@ -463,9 +483,9 @@ __global__ __launch_bounds__(kThreads, 1) void k_linear_dtl(const uint16_t *__re
 
 // Shapes: K % 64 == 0, N % 8 == 0, 16-byte aligned X, W codes and Y, 8-byte aligned bias
 // (checked by the caller).  M, N < 2^31, K < 2^22.  y_st != NULL selects the GELU-statistic
-// epilogue and the settle kernel (scale for y_smax).
+// epilogue and the settle kernel (scale for y_smax).  f32: fp32 outputs (one group, no bias, no y_st).
 static int launch(const uint16_t *x, const uint8_t *w_codes, const Groups &g, const uint16_t *bias, int64_t M,
-                  int64_t N, int64_t K, hif8_stream_t stream, State *y_st, float y_smax)
+                  int64_t N, int64_t K, hif8_stream_t stream, State *y_st, float y_smax, bool f32 = false)
 {
     hipStream_t s = (hipStream_t)stream;
     if (K >= (int64_t(1) << 22)) return HIF8_ERR_SHAPE;
@@ -474,16 +494,16 @@ static int launch(const uint16_t *x, const uint8_t *w_codes, const Groups &g, co
     const int64_t tiles = int64_t(tiles_m) * tiles_n;
     if (tiles >= (int64_t(1) << 31)) return HIF8_ERR_SHAPE;
     if (const int tile = small_linear_tile(M, N, K)) {
-        const int rc = launch_linear_small(tile, x, w_codes, g, bias, M, N, K, y_st, stream);
+        const int rc = launch_linear_small(tile, x, w_codes, g, bias, M, N, K, y_st, f32, stream);
         if (rc != HIF8_OK) return rc;
         return y_st ? launch_gelu_stat_settle(y_st, y_smax, stream) : HIF8_OK;
     }
     if (y_st)
         hipLaunchKernelGGL(dtl::k_linear_dtl<1>, dim3(unsigned(tiles)), dim3(dtl::kThreads), 0, s, x, w_codes, g, bias,
-                           int(M), int(N), int(K), tiles_m, tiles_n, y_st);
+                           int(M), int(N), int(K), tiles_m, tiles_n, y_st, 0);
     else
         hipLaunchKernelGGL(dtl::k_linear_dtl<0>, dim3(unsigned(tiles)), dim3(dtl::kThreads), 0, s, x, w_codes, g, bias,
-                           int(M), int(N), int(K), tiles_m, tiles_n, (State *)nullptr);
+                           int(M), int(N), int(K), tiles_m, tiles_n, (State *)nullptr, f32 ? 1 : 0);
     if (hipGetLastError() != hipSuccess) return HIF8_ERR_HIP;
     return y_st ? launch_gelu_stat_settle(y_st, y_smax, stream) : HIF8_OK;
 }
@@ -498,6 +518,18 @@ int launch_linear_dtl(const uint16_t *x, const uint8_t *w_codes, const State *w_
     g.st[0] = w_st;
     g.y[0] = y;
     return launch(x, w_codes, g, bias, M, N, K, stream, y_st, y_smax);
+}
+
+int launch_linear_dtl_f32(const uint16_t *x, const uint8_t *w_codes, const State *w_st, float *y, int64_t M, int64_t N,
+                          int64_t K, hif8_stream_t stream)
+{
+    Groups g{};
+    g.n = 1;
+    g.tile_end[0] = int((N + dtl::kTile - 1) / dtl::kTile);
+    g.cols[0] = int(N);
+    g.st[0] = w_st;
+    g.y[0] = (uint16_t *)y;
+    return launch(x, w_codes, g, nullptr, M, N, K, stream, nullptr, 0.0f, true);
 }
 
 int launch_linear_dtl_groups(const uint16_t *x, const uint8_t *w_codes, const Groups &g, const uint16_t *bias,

@@ -80,6 +80,7 @@ template <int WM_, int WN_, int MT_, int NT_, int KS_, int S_, bool PIPE_> struc
     static_assert(WM * WN == kWaves && S >= (PIPE ? 3 : 2) && KS >= 1 && !(PIPE && KS > 1) && LDS <= 163840, "tile");
 };
 
+// EPI 1: the GELU statistic of the outputs; 2: fp32 outputs, the sums themselves.
 template <class C, int EPI>
 __global__ __launch_bounds__(kThreads) void k_linear_small(const uint16_t *__restrict__ X, const uint8_t *__restrict__ Wc,
                                                            const Groups G, const uint16_t *__restrict__ bias, int M,
@@ -301,6 +302,23 @@ __global__ __launch_bounds__(kThreads) void k_linear_small(const uint16_t *__res
     barrier();
 
     // Epilogue: acc[i][j] lane (r, g), element e is output n = wn + 16 i + 4 g + e, m = wm + 16 j + r
+    if constexpr (EPI == 2) {
+        // through VGPRs: stored straight from the accumulators' registers, those took part of the loop's
+        // fragments along and the 128 x 128 tile's loop ran 1.5 times its time
+        float *Yf = (float *)Y;
+#pragma unroll
+        for (int i = 0; i < C::NT; ++i) {
+            const int n = n0 + int(wn + uint32_t(i * 16) + 4u * g);
+#pragma unroll
+            for (int j = 0; j < C::MT; ++j) {
+                const int m = m0 + int(wm + uint32_t(j * 16) + r);
+                f32x4 v = acc[i][j];
+                ASMV("" : "+v"(v));
+                if (m < M && n < N) *(f32x4 *)(Yf + size_t(m) * size_t(N) + size_t(n)) = v;
+            }
+        }
+        return;
+    }
     uint8_t *so = smem + kLut;
 #pragma unroll
     for (int i = 0; i < C::NT; ++i) {
@@ -341,7 +359,7 @@ __global__ __launch_bounds__(kThreads) void k_linear_small(const uint16_t *__res
 
 template <class C>
 static int launch(const uint16_t *x, const uint8_t *w, const Groups &g, const uint16_t *bias, int64_t M, int64_t N,
-                  int64_t K, State *y_st, hipStream_t s)
+                  int64_t K, State *y_st, bool f32, hipStream_t s)
 {
     const int tiles_m = int((M + C::TM - 1) / C::TM), tiles_n = int((N + C::TN - 1) / C::TN);
     const int group_m = tiles_m < 8 ? tiles_m : 8;
@@ -349,6 +367,9 @@ static int launch(const uint16_t *x, const uint8_t *w, const Groups &g, const ui
     if (y_st)
         hipLaunchKernelGGL((k_linear_small<C, 1>), grid, dim3(kThreads), 0, s, x, w, g, bias, int(M), int(N), int(K),
                            tiles_m, tiles_n, group_m, y_st);
+    else if (f32)
+        hipLaunchKernelGGL((k_linear_small<C, 2>), grid, dim3(kThreads), 0, s, x, w, g, bias, int(M), int(N), int(K),
+                           tiles_m, tiles_n, group_m, (State *)nullptr);
     else
         hipLaunchKernelGGL((k_linear_small<C, 0>), grid, dim3(kThreads), 0, s, x, w, g, bias, int(M), int(N), int(K),
                            tiles_m, tiles_n, group_m, (State *)nullptr);
@@ -402,15 +423,15 @@ int small_linear_tile(int64_t M, int64_t N, int64_t K)
 }
 
 int launch_linear_small(int tile, const uint16_t *x, const uint8_t *w_codes, const Groups &g, const uint16_t *bias,
-                        int64_t M, int64_t N, int64_t K, State *y_st, hif8_stream_t stream)
+                        int64_t M, int64_t N, int64_t K, State *y_st, bool f32, hif8_stream_t stream)
 {
     using namespace small;
     hipStream_t s = (hipStream_t)stream;
     switch (tile) {
-    case 1: return launch<T32>(x, w_codes, g, bias, M, N, K, y_st, s);
-    case 2: return launch<T64>(x, w_codes, g, bias, M, N, K, y_st, s);
-    case 3: return launch<T128x64>(x, w_codes, g, bias, M, N, K, y_st, s);
-    default: return launch<T128>(x, w_codes, g, bias, M, N, K, y_st, s);
+    case 1: return launch<T32>(x, w_codes, g, bias, M, N, K, y_st, f32, s);
+    case 2: return launch<T64>(x, w_codes, g, bias, M, N, K, y_st, f32, s);
+    case 3: return launch<T128x64>(x, w_codes, g, bias, M, N, K, y_st, f32, s);
+    default: return launch<T128>(x, w_codes, g, bias, M, N, K, y_st, f32, s);
     }
 }
 

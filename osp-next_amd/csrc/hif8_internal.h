@@ -65,10 +65,13 @@ int launch_linear_dtl(const uint16_t *x, const uint8_t *w_codes, const State *w_
                       uint16_t *y, int64_t M, int64_t N, int64_t K, hif8_stream_t stream, State *y_st = nullptr,
                       float y_smax = 0.0f);
 // The same GEMM on small tiles (hif8_gemm_small.hip), equal bit for bit: the tile (1 .. 4) that suits a
-// call, 0 for the 256 x 256 kernel; and its launch (y_st not settled).
+// call, 0 for the 256 x 256 kernel; and its launch (y_st not settled; f32: fp32 outputs).
 int small_linear_tile(int64_t M, int64_t N, int64_t K);
 int launch_linear_small(int tile, const uint16_t *x, const uint8_t *w_codes, const Groups &g, const uint16_t *bias,
-                        int64_t M, int64_t N, int64_t K, State *y_st, hif8_stream_t stream);
+                        int64_t M, int64_t N, int64_t K, State *y_st, bool f32, hif8_stream_t stream);
+// Both with fp32 outputs, the sums themselves, and no bias.
+int launch_linear_dtl_f32(const uint16_t *x, const uint8_t *w_codes, const State *w_st, float *y, int64_t M, int64_t N,
+                          int64_t K, hif8_stream_t stream);
 // The decode-free twin (hif8_gemm_w16.hip): W given as dequantised bf16 [N, K].
 int launch_linear_w16(const uint16_t *x, const uint16_t *w_q, const uint16_t *bias, uint16_t *y, int64_t M,
                       int64_t N, int64_t K, hif8_stream_t stream, State *y_st, float y_smax);

@@ -74,3 +74,16 @@ extern "C" int hif8_linear_fwd(const uint16_t *a, const uint8_t *w_codes, const 
     if (tiles >= (int64_t(1) << 31)) return HIF8_ERR_SHAPE;
     return launch_linear_dtl(a, w_codes, (const State *)w_state, bias, y, M, N, K, stream);
 }
+
+extern "C" int hif8_linear_fwd_f32(const uint16_t *a, const uint8_t *w_codes, const void *w_state, float *y, int64_t M,
+                                   int64_t N, int64_t K, hif8_stream_t stream)
+{
+    if (!a || !w_codes || !w_state || !y) return HIF8_ERR_ARG;
+    if (M <= 0 || N <= 0 || K <= 0) return HIF8_ERR_ARG;
+    if (M >= (int64_t(1) << 31) || N >= (int64_t(1) << 31) || K >= (int64_t(1) << 22)) return HIF8_ERR_SHAPE;
+    if (K % kBK != 0 || N % 8 != 0) return HIF8_ERR_SHAPE;
+    if (((uintptr_t)a | (uintptr_t)w_codes | (uintptr_t)y) & 15u) return HIF8_ERR_ALIGN;
+    const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
+    if (tiles >= (int64_t(1) << 31)) return HIF8_ERR_SHAPE;
+    return launch_linear_dtl_f32(a, w_codes, (const State *)w_state, y, M, N, K, stream);
+}

@@ -327,8 +327,8 @@ def dgrad_fused_ok(grad_q: Tensor, w: "PackedWeight") -> bool:
 
 
 def linear_dgrad(grad_q2: Tensor, w: "PackedWeight", out_dtype: torch.dtype = torch.bfloat16) -> Tensor:
-    """grad_q [M, N] @ w_q [N, K] -> [M, K] bf16 (hif8_linear.py:97; ``out_dtype`` fp32 for the
-    gradient of an fp32 input, on the decode-once route without the rounding to bf16): the forward GEMM with the
+    """grad_q [M, N] @ w_q [N, K] -> [M, K] bf16 (hif8_linear.py:97), or with ``out_dtype`` fp32 (the
+    gradient of an fp32 input) the fp32 sums themselves at every M: the forward GEMM with the
     transposed weight codes [K, N] as its weight, on the route the forward takes at this M (the
     fused GEMM, or the transposed codes decoded once and the decode-free GEMM with its last
     partial wave of tiles split over k ranges).  The reduction (N) is padded to a multiple of 64
@@ -340,21 +340,25 @@ def linear_dgrad(grad_q2: Tensor, w: "PackedWeight", out_dtype: torch.dtype = to
     if Np != N:
         g = pad_2d(g, M, Np)
     codes_t = w.codes_t() if (Np, Kp) == (N, K) else w.codes_t_padded(Kp, Np)
+    f32 = out_dtype == torch.float32
+    L, s = _lib.load(), _lib.stream_ptr(g.device)
     if decode_once(M, Np):
         w_qt = decode(codes_t, w.state, torch.bfloat16)
-        if out_dtype == torch.float32:
+        if f32:
             y = torch.empty((M, Kp), dtype=torch.float32, device=g.device)
             ws, nbytes = _ksplit_workspace(M, Kp, Np, g.device)
-            _lib.check(_lib.load().hif8_linear_fwd_scaled(g.data_ptr(), w_qt.data_ptr(), None, y.data_ptr(),
-                                                          _lib.DTYPE_F32, M, Kp, Np,
-                                                          ws.data_ptr() if ws is not None else None, nbytes,
-                                                          _lib.stream_ptr(g.device)), "hif8_linear_fwd_scaled")
+            _lib.check(L.hif8_linear_fwd_scaled(g.data_ptr(), w_qt.data_ptr(), None, y.data_ptr(), _lib.DTYPE_F32, M,
+                                                Kp, Np, ws.data_ptr() if ws is not None else None, nbytes, s),
+                       "hif8_linear_fwd_scaled")
         else:
             y = linear_fwd_wq_split(g, w_qt)
     else:
-        y = torch.empty((M, Kp), dtype=torch.bfloat16, device=g.device)
-        _lib.check(_lib.load().hif8_linear_fwd(g.data_ptr(), codes_t.data_ptr(), w.state.ptr, None, y.data_ptr(),
-                                               M, Kp, Np, _lib.stream_ptr(g.device)), "hif8_linear_fwd (dgrad)")
+        y = torch.empty((M, Kp), dtype=torch.float32 if f32 else torch.bfloat16, device=g.device)
+        if f32:
+            rc = L.hif8_linear_fwd_f32(g.data_ptr(), codes_t.data_ptr(), w.state.ptr, y.data_ptr(), M, Kp, Np, s)
+        else:
+            rc = L.hif8_linear_fwd(g.data_ptr(), codes_t.data_ptr(), w.state.ptr, None, y.data_ptr(), M, Kp, Np, s)
+        _lib.check(rc, "hif8_linear_fwd (dgrad)")
     y = y if Kp == K else pad_2d(y, M, K)
     return y.to(out_dtype)
 
@@ -504,7 +508,8 @@ def linear_fwd_wq_split(a: Tensor, w_q: Tensor, bias: Optional[Tensor] = None, s
 # element once per 256-row tile of x), "decode_once" decodes it into a bf16 buffer per call and
 # runs the decode-free twin (hif8_linear_fwd_wq), "auto" takes decode_once from
 # DECODE_ONCE_MIN_ROWS rows up, or from DECODE_ONCE_MIN_ROWS_SHORT_K rows up when the reduction
-# depth K is at most SHORT_K.  Both issue the same MFMA products in the same order: the same bits.
+# depth K is at most SHORT_K.  Both issue the same MFMA products in the same order: the same bits
+# (but for the backward's decode-once products, which may add a last wave's k ranges as fp32 partials).
 # Measured fused / decode-once times (decode included; alternating A/B on one box): K = 1536 (the
 # 1.3B q/k/v/o and FFN-up) 0.82-0.98 at 4096-16384 rows, 0.99-1.01 at 32760 (config 2), 1.02-1.03
 # from 49152; K = 5120 or more 0.96-1.01 at 4096-8192 rows, 1.01-1.05 from 16384.

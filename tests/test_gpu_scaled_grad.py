@@ -72,16 +72,24 @@ def test_dgrad_scaled(pkg, M, N, K, out_dtype):
     bound(got, gq, packed.dequantize(torch.float32), out_dtype)
 
 
+# the decode-once route (8192 rows, 24576 where N <= 2048) and the fused one just below it, on its 256 x 256
+# tile and on each small one; ragged rows, padded features and reductions
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(8192, 2112, 40), (8200, 2304, 264), (24600, 64, 8), (8193, 2100, 36), (8192, 2112, 2304)])
+@pytest.mark.parametrize("M,N,K", [(8192, 2112, 40), (8200, 2304, 264), (24600, 64, 8), (8193, 2100, 36),
+                                   (8192, 2112, 2304), (8191, 2112, 40), (8191, 2112, 2304), (24575, 64, 8),
+                                   (4097, 320, 8960), (1, 64, 8), (33, 192, 40), (65, 384, 1544), (300, 256, 2568),
+                                   (1000, 1600, 1536), (257, 100, 36)])
 def test_dgrad_fp32_output(pkg, M, N, K):
-    """The gradient of an fp32 input with a bf16 weight on the decode-once route: fp32, unrounded."""
+    """The gradient of an fp32 input with a bf16 weight: fp32, unrounded, whatever the route."""
     print(f"[scaled] dgrad fp32 M={M} N={N} K={K}", flush=True)
-    assert pkg.hif8_linear.decode_once(M, -(-N // 64) * 64)
     g = torch.Generator().manual_seed(M + N + K)
     gq, _ = pkg._quant(torch.randn(M, N, generator=g).to(torch.bfloat16).to(DEV), 224.0)
     packed = pkg.PackedWeight((torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16).to(DEV), 15.0)
-    bound(pkg.linear_dgrad(gq, packed, torch.float32), gq, packed.dequantize(torch.bfloat16), torch.float32)
+    y = pkg.linear_dgrad(gq, packed, torch.float32)
+    bound(y, gq, packed.dequantize(torch.bfloat16), torch.float32)
+    if not pkg.hif8_linear.decode_once(M, -(-N // 64) * 64):
+        # the bf16 output is these sums rounded
+        assert torch.equal(y.to(torch.bfloat16), pkg.linear_dgrad(gq, packed))
 
 
 @pytest.mark.gpu
@@ -223,6 +231,11 @@ def test_scaled_status_codes_without_gpu(pkg):
     assert wg(g=None) == -1 and wg(st=None) == -1 and wg(dt=2) == -1 and wg(tokens=0) == -1
     assert wg(n=260) == -2 and wg(k=100) == -2 and wg(tokens=1 << 22) == -2 and wg(dw=fake + 2) == -3
     assert fw(a=None) == -1 and fw(dt=3) == -1 and fw(N=0) == -1
+    assert L.hif8_linear_fwd_f32(None, fake, fake, fake, 64, 64, 64, None) == -1
+    assert L.hif8_linear_fwd_f32(fake, fake, fake, fake, 0, 64, 64, None) == -1
+    assert L.hif8_linear_fwd_f32(fake, fake, fake, fake, 64, 100, 64, None) == -2
+    assert L.hif8_linear_fwd_f32(fake, fake, fake, fake, 64, 64, 100, None) == -2
+    assert L.hif8_linear_fwd_f32(fake, fake, fake, fake + 8, 64, 64, 64, None) == -3
     assert fw(K=100) == -2 and fw(N=100) == -2 and fw(K=1 << 22) == -2 and fw(y=fake + 8) == -3
     assert L.hif8_decode_values(None, 16, None, fake, None) == -1
     assert L.hif8_decode_values(fake, 16, None, fake + 4, None) == -3
