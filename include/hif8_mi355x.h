@@ -340,12 +340,18 @@ int hif8_transpose_bf16(const uint16_t *x, int64_t rows, int64_t cols, int64_t r
 int hif8_linear_wgrad(const uint16_t *g, const uint16_t *x, uint16_t *dw, int64_t tokens, int64_t n_out,
                       int64_t k_in, void *workspace, int64_t workspace_bytes, hif8_stream_t stream);
 
-/* Workspace of a wider split: as hif8_linear_split_workspace_bytes, and k ranges also for the grids
- * that leaves whole although they idle CUs (fewer tiles than CUs, or a last wave over half full), where
- * the time they save exceeds the partials' traffic.  hif8_linear_wgrad, hif8_linear_fwd_wq_split and
- * the two entry points below split so when the workspace holds that many bytes (at most 192 MiB on
- * 256 CUs; the 36 tiles of the 1.3B q/k/v/o weight gradient split 7 ways). */
+/* hif8_linear_wgrad and hif8_linear_fwd_wq_split with a wider split: as there, and k ranges also for the
+ * grids they leave whole although these idle CUs (fewer tiles than CUs, or a last wave over half full),
+ * where the time saved exceeds the partials' traffic: 2-32 ranges of at least 8 k-steps.  The workspace
+ * is hif8_linear_ksplit_workspace_bytes (n_out, k_in, tokens or M, N, K) bytes (at most 192 MiB on 256
+ * CUs; the 36 tiles of the 1.3B q/k/v/o weight gradient split 7 ways); with NULL every tile is computed
+ * whole.  The entry point decides the plan, and with it the order of the sums; a larger workspace
+ * changes nothing. */
 int64_t hif8_linear_ksplit_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int hif8_linear_wgrad_ksplit(const uint16_t *g, const uint16_t *x, uint16_t *dw, int64_t tokens, int64_t n_out,
+                             int64_t k_in, void *workspace, int64_t workspace_bytes, hif8_stream_t stream);
+int hif8_linear_fwd_wq_ksplit(const uint16_t *a, const uint16_t *w_q, const uint16_t *bias, uint16_t *y, int64_t M,
+                              int64_t N, int64_t K, void *workspace, int64_t workspace_bytes, hif8_stream_t stream);
 
 /* The backward's products (hif8_linear.py:97,104) where the reference holds one operand in fp32, its
  * quantised values x_q = decode(code) / scale: with that operand given as the HiF8 values themselves,

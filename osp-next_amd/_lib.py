@@ -49,6 +49,8 @@ SIGNATURES = {
     "hif8_linear_split_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "hif8_linear_fwd_wq_split": (_i, [_p, _p, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),
     "hif8_linear_ksplit_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "hif8_linear_fwd_wq_ksplit": (_i, [_p, _p, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),
+    "hif8_linear_wgrad_ksplit": (_i, [_p, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),
     "hif8_linear_wgrad_scaled": (_i, [_p, _p, _p, _p, _i, _i64, _i64, _i64, _p, _i64, _p]),
     "hif8_linear_fwd_scaled": (_i, [_p, _p, _p, _p, _i, _i64, _i64, _i64, _p, _i64, _p]),
     "hif8_decode_values": (_i, [_p, _i64, _p, _p, _p]),

@@ -278,16 +278,15 @@ extern "C" int64_t hif8_linear_ksplit_workspace_bytes(int64_t M, int64_t N, int6
     return plan_ksplit(tiles, K).bytes();
 }
 
-// The split plan that a workspace of workspace_bytes holds: plan_ksplit's, else plan_split's; part NULL
-// where nothing is split.
-static int split_part(void *workspace, int64_t workspace_bytes, int64_t M, int64_t N, int64_t K, float **part,
-                      SplitPlan *plan)
+// The split plan of a call with a workspace: plan_ksplit's where wide, else plan_split's (the entry point
+// says which, never the workspace's size: the sums' order depends on it); part NULL where nothing is split.
+static int split_part(void *workspace, int64_t workspace_bytes, int64_t M, int64_t N, int64_t K, bool wide,
+                      float **part, SplitPlan *plan)
 {
     *part = nullptr;
     if (!workspace) return HIF8_OK;
     const int64_t tiles = ((M + w16::kTile - 1) / w16::kTile) * ((N + w16::kTile - 1) / w16::kTile);
-    *plan = plan_ksplit(tiles, K);
-    if (workspace_bytes < plan->bytes()) *plan = plan_split(tiles, K);
+    *plan = wide ? plan_ksplit(tiles, K) : plan_split(tiles, K);
     if (plan->splits < 2) return HIF8_OK;
     if (workspace_bytes < plan->bytes()) return HIF8_ERR_ARG;
     if ((uintptr_t)workspace & 15u) return HIF8_ERR_ALIGN;
@@ -295,15 +294,14 @@ static int split_part(void *workspace, int64_t workspace_bytes, int64_t M, int64
     return HIF8_OK;
 }
 
-extern "C" int hif8_linear_fwd_wq_split(const uint16_t *a, const uint16_t *w_q, const uint16_t *bias, uint16_t *y,
-                                        int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes,
-                                        hif8_stream_t stream)
+static int fwd_wq_split(const uint16_t *a, const uint16_t *w_q, const uint16_t *bias, uint16_t *y, int64_t M, int64_t N,
+                        int64_t K, void *workspace, int64_t workspace_bytes, bool wide, hif8_stream_t stream)
 {
     int rc = check_w16(a, w_q, bias, y, M, N, K);
     if (rc != HIF8_OK) return rc;
     float *part = nullptr;
     SplitPlan plan{};
-    rc = split_part(workspace, workspace_bytes, M, N, K, &part, &plan);
+    rc = split_part(workspace, workspace_bytes, M, N, K, wide, &part, &plan);
     if (rc != HIF8_OK) return rc;
     Groups g{};
     g.n = 1;
@@ -313,8 +311,22 @@ extern "C" int hif8_linear_fwd_wq_split(const uint16_t *a, const uint16_t *w_q, 
     return launch_w16(a, w_q, g, bias, M, N, K, stream, nullptr, 0.0f, part, false, &plan);
 }
 
-extern "C" int hif8_linear_wgrad(const uint16_t *g, const uint16_t *x, uint16_t *dw, int64_t tokens, int64_t n_out,
-                                 int64_t k_in, void *workspace, int64_t workspace_bytes, hif8_stream_t stream)
+extern "C" int hif8_linear_fwd_wq_split(const uint16_t *a, const uint16_t *w_q, const uint16_t *bias, uint16_t *y,
+                                        int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes,
+                                        hif8_stream_t stream)
+{
+    return fwd_wq_split(a, w_q, bias, y, M, N, K, workspace, workspace_bytes, false, stream);
+}
+
+extern "C" int hif8_linear_fwd_wq_ksplit(const uint16_t *a, const uint16_t *w_q, const uint16_t *bias, uint16_t *y,
+                                         int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes,
+                                         hif8_stream_t stream)
+{
+    return fwd_wq_split(a, w_q, bias, y, M, N, K, workspace, workspace_bytes, true, stream);
+}
+
+static int wgrad(const uint16_t *g, const uint16_t *x, uint16_t *dw, int64_t tokens, int64_t n_out, int64_t k_in,
+                 void *workspace, int64_t workspace_bytes, bool wide, hif8_stream_t stream)
 {
     if (!g || !x || !dw) return HIF8_ERR_ARG;
     if (tokens <= 0 || n_out <= 0 || k_in <= 0) return HIF8_ERR_ARG;
@@ -329,7 +341,7 @@ extern "C" int hif8_linear_wgrad(const uint16_t *g, const uint16_t *x, uint16_t 
     if (tiles >= (int64_t(1) << 31)) return HIF8_ERR_SHAPE;
     float *part = nullptr;
     SplitPlan plan{};
-    const int rc = split_part(workspace, workspace_bytes, n_out, k_in, tokens, &part, &plan);
+    const int rc = split_part(workspace, workspace_bytes, n_out, k_in, tokens, wide, &part, &plan);
     if (rc != HIF8_OK) return rc;
     Groups gr{};
     gr.n = 1;
@@ -337,6 +349,19 @@ extern "C" int hif8_linear_wgrad(const uint16_t *g, const uint16_t *x, uint16_t 
     gr.cols[0] = int(k_in);
     gr.y[0] = dw;
     return launch_w16(g, x, gr, nullptr, n_out, k_in, tokens, stream, nullptr, 0.0f, part, true, &plan);
+}
+
+extern "C" int hif8_linear_wgrad(const uint16_t *g, const uint16_t *x, uint16_t *dw, int64_t tokens, int64_t n_out,
+                                 int64_t k_in, void *workspace, int64_t workspace_bytes, hif8_stream_t stream)
+{
+    return wgrad(g, x, dw, tokens, n_out, k_in, workspace, workspace_bytes, false, stream);
+}
+
+extern "C" int hif8_linear_wgrad_ksplit(const uint16_t *g, const uint16_t *x, uint16_t *dw, int64_t tokens,
+                                        int64_t n_out, int64_t k_in, void *workspace, int64_t workspace_bytes,
+                                        hif8_stream_t stream)
+{
+    return wgrad(g, x, dw, tokens, n_out, k_in, workspace, workspace_bytes, true, stream);
 }
 
 extern "C" int hif8_linear_fwd_wq_gelu_stat(const uint16_t *a, const uint16_t *w_q, const uint16_t *bias,

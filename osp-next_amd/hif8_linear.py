@@ -385,8 +385,8 @@ def wgrad_ok(grad_q2: Tensor, x_q2: Tensor) -> bool:
 
 def linear_wgrad(grad_q2: Tensor, x_q2: Tensor, split_tail: bool = True, transposed: bool = False) -> Tensor:
     """grad_weight = grad_q^T [N, M] @ x_q [M, K] -> [N, K] bf16 (hif8_linear.py:100-105, fp32
-    accumulation): hif8_linear_wgrad, the decode-free GEMM reading both operands token-major as
-    they are, with the last partial wave of tiles split over token ranges unless ``split_tail`` is
+    accumulation): hif8_linear_wgrad_ksplit, the decode-free GEMM reading both operands token-major as
+    they are, with the tiles that would leave CUs idle split over token ranges unless ``split_tail`` is
     False.  Operands too large for its 32-bit offsets (or ``transposed=True``) take the transposed
     route: both operands transposed with the tokens zero-padded to a multiple of 64, then the
     row-major GEMM over the padded tokens (the zeros add nothing)."""
@@ -403,10 +403,10 @@ def linear_wgrad(grad_q2: Tensor, x_q2: Tensor, split_tail: bool = True, transpo
     if not transposed:
         dw = torch.empty((N, K), dtype=torch.bfloat16, device=g.device)
         ws, nbytes = _ksplit_workspace(N, K, M, g.device) if split_tail else (None, 0)
-        rc = L.hif8_linear_wgrad(g.data_ptr(), x.data_ptr(), dw.data_ptr(), M, N, K,
-                                 ws.data_ptr() if ws is not None else None, nbytes, _lib.stream_ptr(g.device))
+        rc = L.hif8_linear_wgrad_ksplit(g.data_ptr(), x.data_ptr(), dw.data_ptr(), M, N, K,
+                                        ws.data_ptr() if ws is not None else None, nbytes, _lib.stream_ptr(g.device))
         if rc != _lib.ERR_SHAPE:
-            _lib.check(rc, "hif8_linear_wgrad")
+            _lib.check(rc, "hif8_linear_wgrad_ksplit")
             return dw
     Mp = (M + 63) // 64 * 64
     g_t = transpose_bf16(g, Mp)
@@ -482,9 +482,10 @@ def linear_dgrad_scaled(grad_q2: Tensor, w: "PackedWeight", out_dtype: torch.dty
 
 def linear_fwd_wq_split(a: Tensor, w_q: Tensor, bias: Optional[Tensor] = None, split_tail: bool = True,
                         wide: bool = False) -> Tensor:
-    """hif8_linear_fwd_wq_split: y = a @ w_q^T (+ bias), bf16, with the tail of the tile grid split
-    over k ranges into a transient fp32 workspace (hif8_linear_split_workspace_bytes, or with
-    ``wide`` hif8_linear_ksplit_workspace_bytes) unless ``split_tail`` is False."""
+    """hif8_linear_fwd_wq_split, or with ``wide`` hif8_linear_fwd_wq_ksplit: y = a @ w_q^T (+ bias), bf16,
+    with the tail of the tile grid split over k ranges into a transient fp32 workspace
+    (hif8_linear_split_workspace_bytes, hif8_linear_ksplit_workspace_bytes) unless ``split_tail`` is
+    False."""
     M, K = a.shape
     N = w_q.shape[0]
     if w_q.shape[1] != K or w_q.dtype != torch.bfloat16 or a.dtype != torch.bfloat16:
@@ -495,12 +496,12 @@ def linear_fwd_wq_split(a: Tensor, w_q: Tensor, bias: Optional[Tensor] = None, s
     if bias is not None:
         bias = _bf16_bias(bias)
         b_ptr = bias.data_ptr()
-    need = L.hif8_linear_ksplit_workspace_bytes if wide else L.hif8_linear_split_workspace_bytes
+    need, name = ((L.hif8_linear_ksplit_workspace_bytes, "hif8_linear_fwd_wq_ksplit") if wide
+                  else (L.hif8_linear_split_workspace_bytes, "hif8_linear_fwd_wq_split"))
     nbytes = int(need(M, N, K)) if split_tail else 0
     ws = torch.empty((nbytes + 3) // 4, dtype=torch.float32, device=a.device) if nbytes > 0 else None
-    _lib.check(L.hif8_linear_fwd_wq_split(a.data_ptr(), w_q.data_ptr(), b_ptr, y.data_ptr(), M, N, K,
-                                          ws.data_ptr() if ws is not None else None, nbytes,
-                                          _lib.stream_ptr(a.device)), "hif8_linear_fwd_wq_split")
+    _lib.check(getattr(L, name)(a.data_ptr(), w_q.data_ptr(), b_ptr, y.data_ptr(), M, N, K,
+                                ws.data_ptr() if ws is not None else None, nbytes, _lib.stream_ptr(a.device)), name)
     return y
 
 

@@ -149,6 +149,27 @@ def test_wgrad_small_grid_split(pkg):
         assert torch.equal(got.view(torch.int16), other.view(torch.int16))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1536, 1536, 4160), (4352, 4096, 1088)])   # 36 tiles; 272: 16 split 2 ways
+def test_workspace_size_does_not_choose_the_sum_order(pkg, M, N, K):
+    """hif8_linear_fwd_wq_split and hif8_linear_wgrad split as hif8_linear_split_workspace_bytes says,
+    however much more a caller's workspace holds: the bits of the exact size (of no workspace where that
+    is 0)."""
+    L, s = pkg._lib.load(), pkg._lib.stream_ptr(torch.device(DEV))
+    g = torch.Generator().manual_seed(M)
+    a, b = (torch.randn(n, K, generator=g).to(torch.bfloat16).to(DEV) for n in (M, N))
+    at, bt = a.t().contiguous(), b.t().contiguous()
+    need, wide = L.hif8_linear_split_workspace_bytes(M, N, K), L.hif8_linear_ksplit_workspace_bytes(M, N, K)
+    assert max(need, wide) > 0
+    ws = torch.empty(max(need, wide) + (1 << 20), dtype=torch.uint8, device=DEV)
+    for fn in (lambda y, p, n: L.hif8_linear_fwd_wq_split(a.data_ptr(), b.data_ptr(), None, y.data_ptr(), M, N, K, p, n, s),
+               lambda y, p, n: L.hif8_linear_wgrad(at.data_ptr(), bt.data_ptr(), y.data_ptr(), K, M, N, p, n, s)):
+        exact, large = (torch.empty(M, N, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        assert fn(exact, ws.data_ptr() if need else None, need) == 0
+        assert fn(large, ws.data_ptr(), ws.numel()) == 0
+        assert torch.equal(exact.view(torch.int16), large.view(torch.int16))
+
+
 def test_ksplit_plan_on_256_cus(pkg):
     """hif8_linear_ksplit_workspace_bytes as planned for 256 CUs (assumed without a GPU): the tails of
     the split-tail plan as they are there, small grids in ranges of at least 8 k-steps, nothing where
