@@ -455,22 +455,28 @@ __global__ __launch_bounds__(TPB) void k_quant(const void *__restrict__ xv, int6
 // The fake quant of a bf16 gradient [rows, cols] (NPU semantics) with the column sums of its result, which
 // are the bias gradient (hif8_linear.py:93,107): a sum over g_q as a pass of its own reads it all again
 // (106 us for [32760, 8960], the copy rate).  A workgroup takes `width` 16-byte chunks of the columns
-// (blockIdx.x) by rpw rows (blockIdx.y): a thread keeps one chunk's 8 columns, its sums in registers,
-// kColRows rows in flight, and leaves them in part[blockIdx.y][cols] for k_colsum_reduce.  The scale
-// comes from the amax pass's parts as in k_quant.  With amax and reduction (us), against hif8_quantize and
+// (blockIdx.x) by `lanes` x rpl rows (blockIdx.y): a thread keeps one chunk's 8 columns over rpl rows,
+// its sums in registers, kColRows rows in flight.  lanes = 256 / width threads share a chunk's column on
+// rows of their own (one where width > 128) and add their sums up in LDS; the workgroup's sums go to
+// part[blockIdx.y][cols] for k_colsum_reduce.  The scale comes from the amax pass's parts as in k_quant.  With amax and reduction (us), against hif8_quantize and
 // torch's sum: [32760, 8960] 326 against 280 + 111, [32760, 1536] 65 against 53 + 39, [75600, 5120] 458 against 366 + 149,
-// [500, 1536] 16 against 11 + 15.  It is bound by its arithmetic and table lookups (5.0 TB/s against the plain pass's 6.1).
+// [500, 1536] 16 against 11 + 15.  Narrow ones with one lane -> their lanes, against hif8_quantize and the sum together:
+// [75600, 64] 94 -> 16 against 30, [32760, 8] 35 -> 17 against 20, [75600, 512] 76 -> 52 against 99.  It is bound by its arithmetic and table lookups (5.0 TB/s against the plain pass's 6.1).
 constexpr int kColRows = 8;
 __global__ __launch_bounds__(kTPB) void k_quant_cols(const uint16_t *__restrict__ x, int64_t rows, int64_t cols,
                                                       State *st, uint16_t *__restrict__ xq, int parts, float smax,
-                                                      int width, int rpw, float *__restrict__ part)
+                                                      int width, int lanes, int rpl, float *__restrict__ part)
 {
     __shared__ __attribute__((aligned(16))) uint8_t lds[kLdsBytes];
+    constexpr uint32_t kSums = kLdsLutF32 + 1024;   // the lanes' sums, between the decode and encode tables
+    static_assert(kSums + kTPB * 8 * 4 <= kTabLo, "LDS map overlap");
+    float *lsum = (float *)(lds + kSums);
     __shared__ uint32_t red[kTPB / 64];
-    const int tid = threadIdx.x;
-    const int64_t cpr = cols >> 3, c = int64_t(blockIdx.x) * width + tid;
-    const bool live = tid < width && c < cpr;
-    const int64_t r0 = int64_t(blockIdx.y) * rpw, r1 = r0 + rpw < rows ? r0 + rpw : rows;
+    const int tid = threadIdx.x, rl = tid / width, cc = tid - rl * width;
+    const int64_t cpr = cols >> 3, c = int64_t(blockIdx.x) * width + cc;
+    const bool live = rl < lanes && c < cpr;
+    const int64_t r0 = (int64_t(blockIdx.y) * lanes + rl) * rpl;
+    const int64_t r1 = !live ? r0 : (r0 + rpl < rows ? r0 + rpl : rows);
     const u32x4 *src = (const u32x4 *)x + c;
     u32x4 *dst = (u32x4 *)xq + c;
     bool fast;
@@ -482,7 +488,6 @@ __global__ __launch_bounds__(kTPB) void k_quant_cols(const uint16_t *__restrict_
         for (uint32_t i = tid; i < sizeof(EncTable) / 16; i += kTPB) d[i] = et[i];
     }
     __syncthreads();
-    if (!live) return;
     const uint16_t *lut16 = (const uint16_t *)(lds + kLdsLutBf16);
     float sum[8] = {};
     for (int64_t r = r0; r < r1; r += kColRows) {
@@ -523,9 +528,26 @@ __global__ __launch_bounds__(kTPB) void k_quant_cols(const uint16_t *__restrict_
             }
         }
     }
-    float *p = part + int64_t(blockIdx.y) * cols + 8 * c;
-    *(float4 *)p = make_float4(sum[0], sum[1], sum[2], sum[3]);
-    *(float4 *)(p + 4) = make_float4(sum[4], sum[5], sum[6], sum[7]);
+    const float4 s0 = make_float4(sum[0], sum[1], sum[2], sum[3]), s1 = make_float4(sum[4], sum[5], sum[6], sum[7]);
+    if (lanes == 1) {
+        if (!live) return;
+        float *p = part + int64_t(blockIdx.y) * cols + 8 * c;
+        *(float4 *)p = s0;
+        *(float4 *)(p + 4) = s1;
+        return;
+    }
+    // one strip of columns (cols = 8 width): the lanes' sums in their order, a column per thread
+    if (live) {
+        float *q = lsum + tid * 8;
+        *(float4 *)q = s0;
+        *(float4 *)(q + 4) = s1;
+    }
+    __syncthreads();
+    for (int k = tid; k < 8 * width; k += kTPB) {
+        float a = 0.0f;
+        for (int l = 0; l < lanes; ++l) a += lsum[l * 8 * width + k];
+        part[int64_t(blockIdx.y) * cols + k] = a;
+    }
 }
 
 // out[c] = sum over b of part[b][c], fp32 or bf16: 32 columns per workgroup, kSumSlots threads a column,
@@ -1241,7 +1263,7 @@ int hif8_quantize_with_codes(const void *x, int dtype, int64_t n, float scale_ma
     return quantize(x, dtype, n, scale_max, state, x_q, HIF8_OUT_BF16, HIF8_SEM_NPU, codes, stream);
 }
 
-// Rows per workgroup of k_quant_cols, a power of two: few enough to fill the chip (500 x 1536: 33 us with
+// Rows per workgroup of k_quant_cols (its least where several lanes share a column), a power of two: few enough to fill the chip (500 x 1536: 33 us with
 // 64 rows, 16 with 16), at most 4096 workgroups and 1024 partials of a column.
 static int colsum_rows(int64_t rows, int64_t strips)
 {
@@ -1269,15 +1291,19 @@ int hif8_quantize_colsum(const uint16_t *x, int64_t rows, int64_t cols, float sc
     if (workspace_bytes < hif8_quantize_colsum_workspace_bytes(rows, cols)) return HIF8_ERR_ARG;
     const int64_t n = rows * cols, strips = colsum_strips(cols);
     const int rpw = colsum_rows(rows, strips);
-    const int64_t blocks = (rows + rpw - 1) / rpw;
-    if (blocks >= 65536) return HIF8_ERR_SHAPE;
+    if ((rows + rpw - 1) / rpw >= 65536) return HIF8_ERR_SHAPE;
     const int width = int(((cols >> 3) + strips - 1) / strips);
+    // rows per thread: rpw or more for the workgroup's lanes together, a multiple of the rows in flight
+    const int lanes = kTPB / width;
+    int rpl = lanes == 1 ? rpw : kColRows;
+    while (int64_t(rpl) * lanes < rpw) rpl *= 2;
+    const int64_t blocks = (rows + int64_t(rpl) * lanes - 1) / (int64_t(rpl) * lanes);
     const int cap = cu_count() * kAmaxWgPerCu;
     const int grid = grid_for((n + 63) / 64, cap < kMaxParts ? cap : kMaxParts);
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL((k_absmax<kBF16, true>), dim3(grid), dim3(kTPB), 0, s, x, n, (State *)state, scale_max);
     hipLaunchKernelGGL(k_quant_cols, dim3(unsigned(strips), unsigned(blocks)), dim3(kTPB), 0, s, x, rows, cols,
-                       (State *)state, x_q, grid, scale_max, width, rpw, (float *)workspace);
+                       (State *)state, x_q, grid, scale_max, width, lanes, rpl, (float *)workspace);
     hipLaunchKernelGGL(k_colsum_reduce, dim3(unsigned((cols + 31) / 32)), dim3(32 * kSumSlots), 0, s, (const float *)workspace,
                        int(blocks), cols, colsum, colsum_dtype == HIF8_DTYPE_F32 ? 1 : 0);
     return last_launch();

@@ -1,7 +1,9 @@
 """hif8_quantize_colsum: the gradient's fake quant with its column sums (the bias gradient,
 hif8_linear.py:93,107) in one pass.  The quantised gradient and the state must equal hif8_quantize's byte
-for byte; the sums lie within 2^-20 of sum |g_q| (fp32 sums of up to 2^13 terms a thread and block, whose
-rounding errors 2^-24 each add at random) of the float64 sums, plus 2^-8 of themselves in bf16."""
+for byte; the sums lie within 2^-20 of sum |g_q| of the float64 sums, plus 2^-8 of themselves in bf16.
+(A column's sum is a chain of at most 128 rows in a thread, at most 256 lanes of a workgroup and 64 of at
+most 1024 workgroups in the shapes here, then 16: under 2^9 fp32 additions, each rounding a partial sum of
+at most sum |g_q| by 2^-24 of it, in either direction; 16 such roundings in one direction are allowed.)"""
 from __future__ import annotations
 
 import pytest
@@ -11,10 +13,13 @@ torch = pytest.importorskip("torch")
 DEV = "cuda:0"
 
 
-# rows around the 8 in flight and the 64 (or more) of a workgroup; columns of one chunk, of part of a
-# strip, of uneven strips; enough of both for larger row blocks
-SHAPES = [(1, 8), (7, 64), (8, 2048), (9, 2056), (63, 1536), (65, 4104), (129, 8960), (1000, 13824), (40000, 2048),
-          (70001, 1536), (300, 40)]
+# rows around the 8 in flight and the 16 (or more) of a workgroup, with partials of several workgroups;
+# columns of one chunk, of part of a strip, of uneven strips; columns that 256, 32, 3 and 2 lanes of a
+# workgroup share (up to 1024 columns), with idle threads beside them and lanes past the last row; enough
+# of both for larger row blocks
+SHAPES = [(1, 8), (7, 64), (8, 2048), (9, 2056), (15, 1536), (16, 1536), (17, 1536), (33, 4104), (63, 1536), (65, 4104),
+          (129, 8960), (1000, 13824), (40000, 2048), (70001, 1536), (300, 40), (2049, 8), (75600, 64), (20001, 680),
+          (5000, 1024), (33000, 1032)]
 
 
 @pytest.mark.gpu
