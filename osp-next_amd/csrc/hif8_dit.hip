@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kThreads) void k_rms_norm_rope(const uint16_t *__re
     }
     for (int64_t row = row0; row < rows; row += wstride) {
         f32x4 ca = {}, sa = {};
-        if (ROPE) {
+        auto rope_row = [&] {
             int64_t cr;
             if (rows <= int64_t(0x7FFFFFFF)) {   // seq divides rows; rep may be larger
                 const uint32_t q = uint32_t(row) / uint32_t(seq), s = uint32_t(row) - q * uint32_t(seq);
@@ -105,7 +105,11 @@ __global__ __launch_bounds__(kThreads) void k_rms_norm_rope(const uint16_t *__re
             const int d = head_dim / 2;
             ca = *(const f32x4 *)(cs + cr * d + pair);
             sa = *(const f32x4 *)(sn + cr * d + pair);
-        }
+        };
+        // ahead of the next row's loads, which they would otherwise wait for; without those, behind the
+        // row's own and its reduction (8192 wide, which one wavefront per SIMD runs: 291 us ahead of the
+        // loads, about 215 behind them; [32760, 8192] rows)
+        if (ROPE && kPre) rope_row();
         u32x4 v[NC];
         const int64_t next = kPre ? row + wstride : row;
         const u32x4 *xr = (const u32x4 *)(x + next * dim);
@@ -128,6 +132,7 @@ __global__ __launch_bounds__(kThreads) void k_rms_norm_rope(const uint16_t *__re
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
         const float r = rsqrtf(ss * inv_dim + eps);
+        if (ROPE && !kPre) rope_row();
         u32x4 *orow = (u32x4 *)(out + row * dim);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {

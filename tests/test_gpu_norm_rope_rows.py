@@ -13,9 +13,9 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# 1, 3, 4 (the last with loads ahead), 5 and 10 chunks a lane; rows: one past the 2048 workgroups' 8192
+# 1, 3, 4 (the last with loads ahead), 5, 10 and 16 chunks a lane; rows: one past the 2048 workgroups' 8192
 # waves, and several turns with a ragged last one
-@pytest.mark.parametrize("dim", [512, 1536, 2048, 2560, 5120])
+@pytest.mark.parametrize("dim", [512, 1536, 2048, 2560, 5120, 8192])
 @pytest.mark.parametrize("seq,batch,rep", [(2731, 3, 1), (2731, 3, 3), (5003, 4, 2), (1, 8193, 8193)])
 @pytest.mark.parametrize("sem", [0, 1])
 def test_rows_in_turn(pkg, dim, seq, batch, rep, sem):
