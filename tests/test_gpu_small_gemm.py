@@ -41,11 +41,18 @@ def test_equals_decode_free(pkg, M, K, N, bias):
 
 @pytest.mark.parametrize("M,K,N", [(1, 64, 8), (64, 320, 264), (300, 256, 2568), (1000, 1600, 1536), (513, 704, 1536)])
 def test_gelu_statistic(pkg, M, K, N):
+    """The outputs and the statistic, wherever in a workgroup's tile the largest output lies."""
     a, _, _, packed, b = operands(pkg, M, K, N, 3 * M + N)
     s_f, s_w = pkg.QuantState(DEV), pkg.QuantState(DEV)
     got = pkg.linear_fwd_gelu_stat(a, packed, b, s_f, 15.0)
     want = pkg.linear_fwd_wq(a, packed.dequantize(torch.bfloat16), b, s_w, 15.0)
     assert same(got, want) and s_f.read() == s_w.read()
+    for at in (0, M // 2, M - 1):
+        top = a.clone()
+        top[at] *= 64
+        pkg.linear_fwd_gelu_stat(top, packed, b, s_f, 15.0)
+        pkg.linear_fwd_wq(top, packed.dequantize(torch.bfloat16), b, s_w, 15.0)
+        assert s_f.read() == s_w.read()
 
 
 @pytest.mark.parametrize("M", [1, 77, 512])
