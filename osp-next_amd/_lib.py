@@ -118,12 +118,15 @@ def check(status: int, what: str) -> None:
 
 
 def stream_ptr(device: torch.device) -> int:
-    """The current stream's handle on a GPU, without building a Stream object (four or more times a
-    linear).  Refuses other devices: a launch would take their pointers as the GPU's."""
-    if device.type != "cuda":
-        raise ValueError(f"the HiF8 path has no CPU route: expected a GPU device, got {device}")
+    """The current stream's handle on a tensor's GPU, without building a Stream object (four or more times
+    a linear).  Refuses host tensors, whose pointers a launch would take as the GPU's; their devices have
+    no index, so that the GPU's, which has one, is not asked for its type (0.2 us)."""
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    if index is None:
+        if device.type != "cuda":
+            raise ValueError(f"the HiF8 path has no CPU route: expected a GPU device, got {device}")
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr(t: torch.Tensor) -> int:
@@ -156,7 +159,7 @@ def unset_state(device: torch.device) -> torch.Tensor:
 def new_state(device: torch.device) -> torch.Tensor:
     """Allocate and initialise one per-tensor quantisation state on ``device``."""
     st = torch.empty(state_size(), dtype=torch.uint8, device=device)
-    check(load().hif8_state_init(ptr(st), stream_ptr(device)), "hif8_state_init")
+    check(load().hif8_state_init(ptr(st), stream_ptr(st.device)), "hif8_state_init")
     return st
 
 

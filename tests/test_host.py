@@ -217,7 +217,7 @@ def test_host_memory_never_reaches_a_launch(pkg, monkeypatch):
         with pytest.raises(ValueError):
             pkg._lib.stream_ptr(torch.device(device))
     a, w = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(8, 64, dtype=torch.bfloat16)
-    for call in (lambda: pkg.QuantState("cpu"), lambda: pkg.linear_fwd_wq(a, w, None),
+    for call in (lambda: pkg.QuantState("cpu"), lambda: pkg.QuantState("cpu:0"), lambda: pkg.linear_fwd_wq(a, w, None),
                  lambda: pkg.hif8_linear.linear_fwd_wq_split(a, w), lambda: pkg.linear_wgrad(a, a)):
         with pytest.raises(ValueError):
             call()
