@@ -568,7 +568,8 @@ static int cu_count()
 // of ranges (150 MB of partials on 256 CUs).  A workgroup takes about 15 us and 2.6 us per 64-key tile;
 // a range's partial costs 0.1 us of the chip to write and add up, and the adding kernel 5 us.  The
 // 1.3B 480P self-attention's 1032 tiles are 4 waves and 8 tiles, which ran a fifth wave alone: 6.65 ->
-// 5.25 ms (990 -> 1255 TFLOP/s).  From 8 waves up the CUs' tile boundaries have drifted apart and the
+// 5.25 ms (990 -> 1255 TFLOP/s).  Over grids of 0.03 to 7.4 waves and 256 to 8192 keys every split one took
+// 0.14 to 0.98 of its whole time.  From 8 waves up the CUs' tile boundaries have drifted apart and the
 // tail fills in by itself (14.4 waves: 1 % slower split).
 struct Plan {
     int full, splits;

@@ -50,7 +50,9 @@ constexpr int kWgPerCu = 3;     // pass 1 (157 VGPRs at dim 5120: 3 wavefronts p
 constexpr int kQdqWgPerCu = 2;  // pass 2 (2 workgroups per CU streamed 1.2-1.4 % faster than 3 at 14B 720P)
 // Pass 1 from per-column extremes (k_modln_amax_ext) keeps one row per wavefront in flight: 2
 // workgroups per CU are best for wide rows (5120: 137 us at 75600 rows, 145 with 4), narrow ones (up to
-// 2048) want more of them in flight (1536, 32760 rows: 34 us with 2, 26 with 4).
+// 2048) want more of them in flight (1536, 32760 rows: 34 us with 2, 26 with 4).  2048 is the widest
+// at which 4 is known to be no slower (48 -> 30 us with the fold's change); 2560 .. 5120 keep the 2 that
+// 5120 was measured with.
 constexpr int ext_wg_per_cu(int nch) { return nch <= 4 ? 4 : 2; }
 
 // Sum over the wavefront, returned to every lane: DPP steps within each row of 16 lanes

@@ -12,9 +12,11 @@ pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
 # one to six 64-k steps (odd counts, steps past the ring's depth), rows and features at and past the
-# edges of the 32 x 32, 64 x 64, 128 x 64 and 128 x 128 tiles, and grids that pick each of them
+# edges of the 32 x 32, 64 x 64, 128 x 64 and 128 x 128 tiles, and grids that pick each of them, the last
+# pairs at and past the rows where the 256 x 256 kernel takes over on 256 CUs
 SHAPES = [(1, 64, 8), (31, 128, 32), (33, 192, 40), (64, 320, 264), (65, 384, 1544), (127, 1024, 2048),
-          (300, 256, 2568), (513, 704, 1536), (260, 448, 8960), (1000, 1600, 1536), (600, 640, 5128), (129, 8960, 776)]
+          (300, 256, 2568), (513, 704, 1536), (260, 448, 8960), (1000, 1600, 1536), (600, 640, 5128), (129, 8960, 776),
+          (2688, 1536, 1536), (2689, 1536, 1536), (384, 1536, 8960), (385, 1536, 8960)]
 
 
 def operands(pkg, M, K, N, seed, bias=True):
